@@ -3,16 +3,13 @@
 // (dA = dC B^T, dB = A^T dC) and a deterministic split-K for tall-skinny
 // products such as the convolution weight gradients.
 //
-// Tiling. A workgroup computes a BM x BN tile of C with (BM/WM) x (BN/WN)
-// wavefronts; each wavefront owns a WM x WN sub-tile made of 32 x 32 blocks
-// accumulated with v_mfma_f32_32x32x2f32 (64 lanes, K = 2 per instruction,
-// 16 fp32 accumulators per lane per block). K advances BK at a time through
-// two LDS buffers laid out [k][m] and [k][n], so every MFMA operand fetch
-// is one conflict-free ds_read_b32 per lane; the next tile's global loads
-// are issued before the current tile's MFMAs and land in the other buffer,
-// one barrier per K step.
+// Tiling. Products large enough for staged tiles run gemm_kernel (gemm_split.hpp): fp32
+// operands split into three bf16 parts while a tile is staged in LDS, six part products on
+// v_mfma_f32_16x16x32_bf16, fp32 accumulation. Products with outputs too small to fill the
+// chip that way run the fp32 instructions: K-sliced 32 x 32 tiles (gemm_kslice,
+// gemm_kernel.hpp), 16 x 16 panels of a long K, and the vector kernels of the smallest.
 //
-// MFMA register layouts (CDNA3/CDNA4 ISA, v_mfma_f32_32x32x2f32):
+// MFMA register layout of the fp32 tiles (CDNA3/CDNA4 ISA, v_mfma_f32_32x32x2f32):
 //   A operand: lane l holds A[i = l % 32][k = l / 32]
 //   B operand: lane l holds B[k = l / 32][j = l % 32]
 //   D result : lane l, register r holds D[8 (r / 4) + 4 (l / 32) + r % 4][l % 32]
@@ -32,7 +29,7 @@
 #include <mutex>
 #include <vector>
 
-#include "gemm_kernel.hpp"
+#include "gemm_split.hpp"
 
 namespace ehip {
 namespace gemm_detail {
@@ -173,31 +170,82 @@ struct Workspace {
 // The grid's z extent: products beyond it run as further launches.
 constexpr int64_t kGridZ = 65535;
 
-// pipe: run the tiles as gemm_nt_pipe (whole 128 x 128 tiles of a batch-1
-// A B^T product; the same split and the same sums as the staged kernel).
-template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB>
-int launch_cfg(const GemmArgs& g0, int64_t batch, bool check, hipStream_t s,
-               const Workspace& wsp, bool pipe = false) {
-    using C = Cfg<BM, BN, BK, WM, WN>;
+// The staged tiles' shapes (gemm_kernel). per_cu: how many of a shape's workgroups a CU holds
+// (LDS and registers); rate: the throughput of a full CU relative to the first shape's,
+// measured on MI355X at 8192 x 1024 x 4096 and 4096^3 (224, 199, 177 and 150 TFLOP/s).
+struct TileShape {
+    int bm, bn, per_cu;
+    double rate;
+};
+constexpr TileShape kShapes[] = {{256, 128, 1, 1.0}, {128, 128, 2, 0.9}, {128, 64, 3, 0.78},
+                                 {64, 64, 3, 0.6}};
+// What is left of a CU's rate when it holds c of a shape's per_cu workgroups: alone, a
+// workgroup has nothing to run in its load and conversion phases (1999 x 1531 x 777 in 192
+// workgroups of 128 x 128: 56 us, in 576 of a third of K each: 46 us).
+double share(int c, int per_cu) {
+    if (c >= per_cu) return 1.0;
+    return c == 1 ? (per_cu == 2 ? 0.65 : 0.5) : 0.8;
+}
+
+// The shape with the least estimated time for an m x n output in `copies` products and K
+// splits: whole rounds of the chip's 256 CUs, then the last one's workgroups spread over
+// them. Every shape forms an element by the same chain of instructions, so the choice does
+// not change a bit.
+int choose_shape(int64_t m, int64_t n, int64_t copies) {
+    int best = 0;
+    double best_t = 0.0;
+    for (int i = 0; i < int(sizeof(kShapes) / sizeof(kShapes[0])); ++i) {
+        const TileShape& t = kShapes[i];
+        const int64_t work = ceil_div(m, t.bm) * ceil_div(n, t.bn) * copies;
+        const int64_t slots = int64_t(256) * t.per_cu;
+        const double unit = double(t.bm) * t.bn / t.rate;
+        const int last = int(ceil_div(work % slots, 256));
+        double time = double(work / slots) * t.per_cu * unit;
+        if (last > 0) time += last * unit / share(last, t.per_cu);
+        if (i == 0 || time < best_t) {
+            best = i;
+            best_t = time;
+        }
+    }
+    return best;
+}
+
+template <int BM, int BN, int WM, int WN, int STAGES, int MINW, bool TA, bool TB>
+int launch_shape(const GemmArgs& g, const dim3& grid, hipStream_t s) {
+    constexpr int kThreads = TileThreads<BM, BN, WM, WN>::value;
+    if constexpr (!TB) {  // column sums exist only for a K x N B
+        if (g.colsum != nullptr) {
+            EHIP_LAUNCH("gemm", (gemm_kernel<BM, BN, WM, WN, STAGES, MINW, TA, TB, true>), grid,
+                        dim3(kThreads), 0, s, g);
+            return EHIP_OK;
+        }
+    }
+    EHIP_LAUNCH("gemm", (gemm_kernel<BM, BN, WM, WN, STAGES, MINW, TA, TB, false>), grid,
+                dim3(kThreads), 0, s, g);
+    return EHIP_OK;
+}
+
+// A product as staged tiles. The K split is planned on bm x bn tiles of bk (the planner's
+// class), whatever shape then runs: its number fixes the order of the sums and the
+// workspace.
+template <bool TA, bool TB>
+int launch_staged(const GemmArgs& g0, int64_t batch, int bm, int bn, int bk, hipStream_t s,
+                  const Workspace& wsp) {
     GemmArgs g = g0;
-    g.tiles_m = int(ceil_div(g.m, BM));
-    g.tiles_n = int(ceil_div(g.n, BN));
-    const int64_t tiles = int64_t(g.tiles_m) * g.tiles_n;
-    // Split K when the tile grid alone cannot fill the chip and K is long:
-    // aim for ~512 workgroups, each at least 8 K steps long. "Fill" is one
-    // workgroup per CU (256) for the 256 x 256 tile, which runs one per CU,
-    // and two per CU (512) for the smaller tiles, which run two or more (a
-    // 1024 x 4096 x 8192 weight gradient: 600 -> 544 us with two splits).
-    const int64_t fill = BM * BN >= 256 * 256 ? 256 : 512;
+    // Split K when the tile grid alone cannot fill the chip and K is long: aim for ~512
+    // workgroups, each at least 8 K steps long. "Fill" is 256 workgroups of the largest
+    // class and two per CU (512) of the smaller ones.
+    const int64_t class_tiles = ceil_div(g.m, bm) * ceil_div(g.n, bn) * batch;
+    const int64_t fill = bm * bn >= 256 * 256 ? 256 : 512;
     int splits = 1;
-    if (tiles * batch < fill && g.k >= 16 * BK) {
-        int64_t want = ceil_div(512, tiles * batch);
-        const int64_t max_by_k = g.k / (8 * BK);
+    if (class_tiles < fill && g.k >= 16 * bk) {
+        int64_t want = ceil_div(512, class_tiles);
+        const int64_t max_by_k = g.k / (8 * bk);
         if (want > max_by_k) want = max_by_k;
         if (want > 256) want = 256;
         if (want > 1) splits = int(want);
     }
-    g.k_chunk = ceil_div(ceil_div(g.k, splits), BK) * BK;
+    g.k_chunk = ceil_div(ceil_div(g.k, splits), kSplitBK) * kSplitBK;
     splits = int(ceil_div(g.k, g.k_chunk));
     g.splits = splits;
     // Unstored tiles would leave their split-K partials unwritten for the
@@ -221,35 +269,25 @@ int launch_cfg(const GemmArgs& g0, int64_t batch, bool check, hipStream_t s,
         }
         g.c = ws;
     }
-    const bool epi = splits == 1 && !plain_epilogue(g);
+    // Causal products skip by row bands of the tile: they keep the class's shape.
+    const int shape = g.causal == 0 ? choose_shape(g.m, g.n, batch * splits)
+                      : bm == 64    ? 3
+                      : bn == 64    ? 2
+                                    : 1;
+    g.tiles_m = int(ceil_div(g.m, kShapes[shape].bm));
+    g.tiles_n = int(ceil_div(g.n, kShapes[shape].bn));
+    const int64_t tiles = int64_t(g.tiles_m) * g.tiles_n;
     // Split K only below ~512 workgroups, so a split product is one launch;
     // longer batches run in ranges of the grid's z extent.
     for (int64_t z0 = 0; z0 < batch; z0 += kGridZ) {
         g.batch0 = z0;
         const dim3 grid{unsigned(tiles), unsigned(splits),
                         unsigned(batch - z0 < kGridZ ? batch - z0 : kGridZ)};
-        if constexpr (BM == 128 && BN == 128 && BK == kNtBK && !TA && TB) {
-            if (pipe) {
-                if (epi)
-                    EHIP_LAUNCH("gemm", gemm_nt_pipe<true>, grid, dim3(256), 0, s, g);
-                else
-                    EHIP_LAUNCH("gemm", gemm_nt_pipe<false>, grid, dim3(256), 0, s, g);
-                continue;
-            }
-        }
-        if (check && epi) {
-            EHIP_LAUNCH("gemm", (gemm_kernel<BM, BN, BK, WM, WN, TA, TB, true, true>), grid,
-                        dim3(C::kThreads), 0, s, g);
-        } else if (check) {
-            EHIP_LAUNCH("gemm", (gemm_kernel<BM, BN, BK, WM, WN, TA, TB, true, false>), grid,
-                        dim3(C::kThreads), 0, s, g);
-        } else if (epi) {
-            EHIP_LAUNCH("gemm", (gemm_kernel<BM, BN, BK, WM, WN, TA, TB, false, true>), grid,
-                        dim3(C::kThreads), 0, s, g);
-        } else {
-            EHIP_LAUNCH("gemm", (gemm_kernel<BM, BN, BK, WM, WN, TA, TB, false, false>), grid,
-                        dim3(C::kThreads), 0, s, g);
-        }
+        const int rc = shape == 0   ? launch_shape<256, 128, 64, 64, 2, 2, TA, TB>(g, grid, s)
+                       : shape == 1 ? launch_shape<128, 128, 64, 32, 1, 4, TA, TB>(g, grid, s)
+                       : shape == 2 ? launch_shape<128, 64, 64, 32, 1, 3, TA, TB>(g, grid, s)
+                                    : launch_shape<64, 64, 32, 32, 2, 3, TA, TB>(g, grid, s);
+        if (rc) return rc;
     }
     if (splits > 1) {
         GemmArgs gr = g0;  // the caller's output and epilogue, the workspace geometry
@@ -322,14 +360,11 @@ int launch_kslice(GemmArgs g, int64_t batch, hipStream_t s) {
     }
 }
 
-// Tile choice, largest first (measured on MI355X, fp32 MFMA):
-//   L  256 x 256 x 16, 8 waves of 128 x 64   ~135 TFLOP/s at 4096^3
-//   M  128 x 128 x 32, 8 waves of  64 x 32   ~120-130 on 8192 x 1024 x K
-//   S  128 x  64 x 32, 8 waves of  32 x 32   thin outputs (N = 64 attention products)
+// Tile classes, largest first:
+//   L, M, S, T  staged tiles, whose K split is planned on 256 x 256, 128 x 128, 128 x 64 and
+//      64 x 64 tiles; launch_staged then picks the shape that runs
 //   K  32 x 32 per workgroup, K sliced over its waves: outputs too small for
 //      the larger tiles to fill the chip (512^3, the char-Transformer's layers)
-//   T   64 x  64 x 16, 4 waves of  32 x 32   the rest (few tiles; B column sums;
-//      products that skip K causally)
 //   P   16 x 16 per workgroup of 16 waves, each wave a sixteenth of K: A^T B
 //       products of few tiles over a long K (weight gradients of narrow
 //       layers), one load round trip per 128 k of a wave, no workspace
@@ -556,31 +591,13 @@ int gemm_modes(GemmArgs g, int64_t batch, hipStream_t s, const Workspace& wsp) {
     // rows are aligned.
     g.vec = operands_aligned(g) ? 1 : 0;
     g.vec_ab = operand_alignment(g);
-    const auto whole = [&](int bm, int bn, int bk) {
-        return g.vec && g.m % bm == 0 && g.n % bn == 0 && g.k % bk == 0;
-    };
-    const Tile tile = plan_tile(g, batch, TA, TB);
-    if constexpr (!TA && TB) {
-        // A B^T in whole 128 x 128 tiles: the two-step pipeline (same sums).
-        if ((tile == Tile::M || tile == Tile::L) && batch == 1 && g.causal == 0 && g.vec &&
-            g.m % 128 == 0 && g.n % 128 == 0 && g.k % kNtBK == 0 &&
-            (g.m / 128) * (g.n / 128) <= 0x7fffffff)
-            return launch_cfg<128, 128, 32, 64, 32, false, true>(g, batch, false, s, wsp, true);
-    }
-    switch (tile) {
-        case Tile::L:
-            return launch_cfg<256, 256, 16, 128, 64, TA, TB>(g, batch, !whole(256, 256, 16), s,
-                                                             wsp);
-        case Tile::M:
-            return launch_cfg<128, 128, 32, 64, 32, TA, TB>(g, batch, !whole(128, 128, 32), s, wsp);
-        case Tile::S:
-            return launch_cfg<128, 64, 32, 32, 32, TA, TB>(g, batch, !whole(128, 64, 32), s, wsp);
-        case Tile::K:
-            return launch_kslice<TA, TB>(g, batch, s);
-        case Tile::P:
-            return launch_panel(g, s);
-        default:
-            return launch_cfg<64, 64, 16, 32, 32, TA, TB>(g, batch, !whole(64, 64, 16), s, wsp);
+    switch (plan_tile(g, batch, TA, TB)) {
+        case Tile::L: return launch_staged<TA, TB>(g, batch, 256, 256, 16, s, wsp);
+        case Tile::M: return launch_staged<TA, TB>(g, batch, 128, 128, 32, s, wsp);
+        case Tile::S: return launch_staged<TA, TB>(g, batch, 128, 64, 32, s, wsp);
+        case Tile::K: return launch_kslice<TA, TB>(g, batch, s);
+        case Tile::P: return launch_panel(g, s);
+        default: return launch_staged<TA, TB>(g, batch, 64, 64, 16, s, wsp);
     }
 }
 
@@ -1030,16 +1047,16 @@ int check_desc(const ehip_gemm_ex_t& d) {
 }
 
 const OccupancyKernel kGemmKernels[] = {
-    {"gemm_kernel 256x256x16, 8 waves of 128x64 (NN)",
-     reinterpret_cast<const void*>(&gemm_kernel<256, 256, 16, 128, 64, false, false, false, false>), 512},
-    {"gemm_kernel 128x128x32, 8 waves of 64x32 (TN: dW)",
-     reinterpret_cast<const void*>(&gemm_kernel<128, 128, 32, 64, 32, true, false, false, false>), 512},
-    {"gemm_kernel 128x128x32 (NT: dX, [row][k] tiles)",
-     reinterpret_cast<const void*>(&gemm_kernel<128, 128, 32, 64, 32, false, true, false, false>), 512},
-    {"gemm_kernel 128x64x32, 8 waves of 32x32 (NN)",
-     reinterpret_cast<const void*>(&gemm_kernel<128, 64, 32, 32, 32, false, false, false, false>), 512},
-    {"gemm_kernel 64x64x16 checked, 4 waves (NN)",
-     reinterpret_cast<const void*>(&gemm_kernel<64, 64, 16, 32, 32, false, false, true, false>), 256},
+    {"gemm_kernel 256x128x32, 8 waves of 64x64 (NN)",
+     reinterpret_cast<const void*>(&gemm_kernel<256, 128, 64, 64, 2, 2, false, false, false>), 512},
+    {"gemm_kernel 256x128x32, 8 waves of 64x64 (TN: dW)",
+     reinterpret_cast<const void*>(&gemm_kernel<256, 128, 64, 64, 2, 2, true, false, false>), 512},
+    {"gemm_kernel 128x128x32, 8 waves of 64x32 (NT)",
+     reinterpret_cast<const void*>(&gemm_kernel<128, 128, 64, 32, 1, 4, false, true, false>), 512},
+    {"gemm_kernel 128x64x32, 4 waves of 64x32 (NN)",
+     reinterpret_cast<const void*>(&gemm_kernel<128, 64, 64, 32, 1, 3, false, false, false>), 256},
+    {"gemm_kernel 64x64x32, 4 waves of 32x32 (TN)",
+     reinterpret_cast<const void*>(&gemm_kernel<64, 64, 32, 32, 2, 3, true, false, false>), 256},
     {"gemm_kslice 32x32, 8 waves (NN)",
      reinterpret_cast<const void*>(&gemm_kslice<8, false, false, false, false>), 512},
     {"gemm_tn_panel 16x16 (TN: narrow dW)",

@@ -253,351 +253,6 @@ __device__ __forceinline__ void store_acc(const GemmArgs& g, floatx16 (&acc)[C::
         }
 }
 
-// Products with both operands stored k-contiguous (A untransposed, B
-// transposed: C = A B^T) keep each operand tile in LDS as [row][k] (row pitch
-// BK + 4), written with one float4 per loaded float4 and read back as one
-// float4 per lane per 8 k. MFMA order inside a block of 8 k at kb: half h of
-// the lanes holds k = kb + 4h + j and instruction j = 0..3 multiplies them.
-// The other layouts ([k][row], above) transpose k-contiguous operands with
-// four scalar LDS writes that conflict on the banks; measured on MI355X this
-// layout runs the NT products of the cfg5 Transformer 8-12 % faster, while
-// for operands stored row-contiguous it is no faster than [k][row], which
-// therefore stays for them.
-template <int BK>
-struct KcTile {
-    static constexpr int kPitch = BK + 4;
-};
-
-// Stores load_tile<..., TRANS = false> registers (row q / (BK / 4), k 4 (q %
-// (BK / 4))) into a [row][k] tile.
-template <class C, int BR, int BK>
-__device__ __forceinline__ void store_tile_kc(float* __restrict__ s, const float4* reg, int loads,
-                                              int total) {
-#pragma unroll
-    for (int i = 0; i < loads; ++i) {
-        const int q = threadIdx.x + i * C::kThreads;
-        if (q < total) {
-            const int r = q / (BK / 4), kk = 4 * (q % (BK / 4));
-            *reinterpret_cast<float4*>(s + r * KcTile<BK>::kPitch + kk) = reg[i];
-        }
-    }
-}
-
-template <class C, int BK>
-__device__ __forceinline__ void mfma_stage_kc(floatx16 (&acc)[C::kFM][C::kFN], const float* lds_a,
-                                              const float* lds_b, int wm0, int wn0, int lane) {
-    constexpr int P = KcTile<BK>::kPitch;
-    static_assert(BK % 8 == 0, "BK");
-    const float* sa = lds_a + (wm0 + lane % 32) * P + 4 * (lane / 32);
-    const float* sb = lds_b + (wn0 + lane % 32) * P + 4 * (lane / 32);
-    float4 fa[2][C::kFM], fb[2][C::kFN];
-#pragma unroll
-    for (int i = 0; i < C::kFM; ++i) fa[0][i] = *reinterpret_cast<const float4*>(sa + 32 * i * P);
-#pragma unroll
-    for (int j = 0; j < C::kFN; ++j) fb[0][j] = *reinterpret_cast<const float4*>(sb + 32 * j * P);
-#pragma unroll
-    for (int kb = 0; kb < BK; kb += 8) {
-        const int f = (kb / 8) & 1;
-        if (kb + 8 < BK) {
-#pragma unroll
-            for (int i = 0; i < C::kFM; ++i)
-                fa[f ^ 1][i] = *reinterpret_cast<const float4*>(sa + 32 * i * P + kb + 8);
-#pragma unroll
-            for (int j = 0; j < C::kFN; ++j)
-                fb[f ^ 1][j] = *reinterpret_cast<const float4*>(sb + 32 * j * P + kb + 8);
-        }
-        if (C::kPrio) __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int i = 0; i < C::kFM; ++i)
-#pragma unroll
-                for (int j = 0; j < C::kFN; ++j) {
-                    const float a = q == 0 ? fa[f][i].x : q == 1 ? fa[f][i].y : q == 2 ? fa[f][i].z : fa[f][i].w;
-                    const float b = q == 0 ? fb[f][j].x : q == 1 ? fb[f][j].y : q == 2 ? fb[f][j].z : fb[f][j].w;
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc[i][j], 0, 0, 0);
-                }
-        if (C::kPrio) __builtin_amdgcn_s_setprio(0);
-    }
-}
-
-// EPI: the fused epilogue (alpha, addend, beta, ReLU); without it the
-// accumulators are stored as they are (also the split-K partials).
-template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, bool CHECK, bool EPI>
-__global__ __launch_bounds__((Cfg<BM, BN, BK, WM, WN>::kThreads)) void gemm_kernel(GemmArgs g) {
-    using C = Cfg<BM, BN, BK, WM, WN>;
-    constexpr bool KC = !TA && TB;  // both operands k-contiguous: [row][k] tiles
-    constexpr int kFloatsA = KC ? BM * KcTile<BK>::kPitch : BK * C::kLdsA;
-    constexpr int kFloatsB = KC ? BN * KcTile<BK>::kPitch : BK * C::kLdsB;
-    __shared__ float lds_a[2][kFloatsA];
-    __shared__ float lds_b[2][kFloatsB];
-
-    // Tile coordinates: XCD-contiguous renumbering, then GROUP_M-row groups.
-    const int tiles = g.tiles_m * g.tiles_n;
-    int tm, tn;
-    int64_t batch = g.batch0 + blockIdx.z;
-    if (g.causal != 0 && gridDim.y == 1) {
-        // Causal skipping makes a tile's work depend on its row band. Workgroups
-        // reach the XCDs (and their CUs) in turn in launch order, so the order
-        // runs over the products first: every XCD and CU then gets tiles of
-        // every band instead of, with few tiles per product, one band only.
-        const int64_t lin = int64_t(blockIdx.z) * gridDim.x + blockIdx.x;
-        batch = g.batch0 + lin % gridDim.z;
-        const int t = int(lin / gridDim.z);
-        tm = t / g.tiles_n;
-        tn = t % g.tiles_n;
-    } else {
-        int bid = blockIdx.x;
-        if (tiles % 8 == 0) bid = (bid % 8) * (tiles / 8) + bid / 8;
-        constexpr int kGroupM = 8;
-        const int group = bid / (kGroupM * g.tiles_n);
-        const int first_m = group * kGroupM;
-        const int gsz = min(g.tiles_m - first_m, kGroupM);
-        const int in_group = bid % (kGroupM * g.tiles_n);
-        tm = first_m + in_group % gsz;
-        tn = in_group / gsz;
-    }
-
-    const int split = blockIdx.y;
-    const float* A = g.a + batch_offset(batch, g.inner, g.stride_a, g.stride_a2);
-    const float* B = g.b + batch_offset(batch, g.inner, g.stride_b, g.stride_b2);
-    const int64_t m0 = int64_t(tm) * BM, n0 = int64_t(tn) * BN;
-    int64_t k_begin = int64_t(split) * g.k_chunk;
-    int64_t k_end = k_begin + g.k_chunk;
-    if (k_end > g.k) k_end = g.k;
-    // Causal skipping (modes of ehip_gemm_ex_t::causal); m0 and m0 + BM are
-    // multiples of BK, so the K steps stay aligned.
-    if (g.causal == 4 && n0 >= m0 + BM) return;  // wholly above the diagonal: not stored
-    if (g.causal == 1 && n0 >= m0 + BM) {
-        k_end = k_begin;  // wholly above the diagonal: the epilogue of acc = 0
-    } else if (g.causal == 2) {
-        if (k_end > m0 + BM) k_end = k_begin > m0 + BM ? k_begin : m0 + BM;
-    } else if (g.causal == 3) {
-        if (k_begin < m0) k_begin = k_end < m0 ? k_end : m0;
-    }
-
-    const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-    const int wm0 = (wave / C::kWavesN) * WM, wn0 = (wave % C::kWavesN) * WN;
-
-    floatx16 acc[C::kFM][C::kFN];
-#pragma unroll
-    for (int i = 0; i < C::kFM; ++i)
-#pragma unroll
-        for (int j = 0; j < C::kFN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-    float4 ra[C::kALoads], rb[C::kBLoads];
-    // The step count is the same for the whole workgroup; read as a scalar so
-    // that the per-step conditions are scalar branches, not exec masks.
-    const int64_t steps = __builtin_amdgcn_readfirstlane(int((k_end - k_begin + BK - 1) / BK));
-    const bool colsum_tile = g.colsum != nullptr && tm == 0;
-    float csum = 0.0f;
-    if (steps > 0) {
-        load_tile<C, BM, BK, TA, CHECK>(A, g.lda, g.m, k_end, m0, k_begin, ra, C::kALoads, C::kA4, g.vec);
-        load_tile<C, BN, BK, !TB, CHECK>(B, g.ldb, g.n, k_end, n0, k_begin, rb, C::kBLoads, C::kB4, g.vec);
-        if constexpr (KC) {
-            store_tile_kc<C, BM, BK>(lds_a[0], ra, C::kALoads, C::kA4);
-            store_tile_kc<C, BN, BK>(lds_b[0], rb, C::kBLoads, C::kB4);
-        } else {
-            store_tile<C, BM, BK, C::kLdsA, TA>(lds_a[0], ra, C::kALoads, C::kA4);
-            store_tile<C, BN, BK, C::kLdsB, !TB>(lds_b[0], rb, C::kBLoads, C::kB4);
-        }
-        __syncthreads();
-    }
-    for (int64_t s = 0; s < steps; ++s) {
-        const int cur = int(s & 1);
-        const bool more = s + 1 < steps;
-        if (more) {
-            const int64_t kn = k_begin + (s + 1) * BK;
-            load_tile<C, BM, BK, TA, CHECK>(A, g.lda, g.m, k_end, m0, kn, ra, C::kALoads, C::kA4, g.vec);
-            load_tile<C, BN, BK, !TB, CHECK>(B, g.ldb, g.n, k_end, n0, kn, rb, C::kBLoads,
-                                             C::kB4, g.vec);
-        }
-        if constexpr (KC)
-            mfma_stage_kc<C, BK>(acc, lds_a[cur], lds_b[cur], wm0, wn0, lane);
-        else
-            mfma_stage<C, BK>(acc, lds_a[cur], lds_b[cur], wm0, wn0, lane);
-        // Column sums exist only for a K x N B (the entry point refuses them
-        // otherwise), so the k-contiguous tiles carry no code for them.
-        if constexpr (!KC) {
-            if (colsum_tile && threadIdx.x < BN) {
-                // This K step's B rows, in k order, for column n0 + threadIdx.x.
-                const float* col = lds_b[cur] + threadIdx.x;
-                float part = 0.0f;
-#pragma unroll
-                for (int kk = 0; kk < BK; ++kk) part += col[kk * C::kLdsB];
-                csum = csum + part;
-            }
-        }
-        if (more) {
-            if constexpr (KC) {
-                store_tile_kc<C, BM, BK>(lds_a[cur ^ 1], ra, C::kALoads, C::kA4);
-                store_tile_kc<C, BN, BK>(lds_b[cur ^ 1], rb, C::kBLoads, C::kB4);
-            } else {
-                store_tile<C, BM, BK, C::kLdsA, TA>(lds_a[cur ^ 1], ra, C::kALoads, C::kA4);
-                store_tile<C, BN, BK, C::kLdsB, !TB>(lds_b[cur ^ 1], rb, C::kBLoads, C::kB4);
-            }
-        }
-        __syncthreads();
-    }
-
-    if (!KC && colsum_tile && threadIdx.x < BN && n0 + threadIdx.x < g.n) {
-        if (g.splits > 1)
-            g.c[int64_t(split) * g.ws_stride + g.m * g.n + n0 + threadIdx.x] = csum;
-        else
-            g.colsum[n0 + threadIdx.x] = csum;
-    }
-
-    // Epilogue. With splits > 1, c is the workspace [split][batch][m][n]
-    // (ws_stride floats per split) and the epilogue is applied by the
-    // reduction kernel.
-    float* Cp;
-    int64_t ldc;
-    if (g.splits > 1) {
-        Cp = g.c + int64_t(split) * g.ws_stride + batch * g.m * g.n;
-        ldc = g.n;
-    } else {
-        Cp = g.c + batch_offset(batch, g.inner, g.stride_c, g.stride_c2);
-        ldc = g.ldc;
-    }
-    const float* addp = g.add ? g.add + (int64_t(batch) % g.add_period) * g.stride_add : nullptr;
-    store_acc<C, CHECK, EPI>(g, acc, Cp, ldc, addp, m0, n0, wm0, wn0, lane);
-}
-
-// ------------------------------------------------------------ NT pipeline
-//
-// C = A B^T with both operands stored k-contiguous (the input gradients dX =
-// dY W^T of Linear layers), whole 128 x 128 tiles, batch 1: four waves of 64 x
-// 64 (2 x 2 blocks of 32 x 32) and the loads two K steps ahead of the MFMAs
-// -- step s + 1 waits in registers while step s runs, is written into the
-// free LDS stage a quarter of the way into step s, and step s + 2's loads are
-// issued right after -- instead of the staged kernel's one step ahead with
-// eight waves. The [row][k] tiles and the MFMA sequence are the staged
-// kernel's (blocks of 8 k ascending, k and k + 4 paired; mfma_stage_kc), and
-// the K split is the one launch_cfg gives a 128 x 128 tile, so each output is
-// the same chain with the same bits; measured on MI355X 5-7 % faster on the
-// cfg5 input-gradient shapes (8192 x 1024 x 1024: 147 against 155 us;
-// 8192 x 1024 x 4096: 505 against 543).
-constexpr int kNtBK = 32;
-typedef float nt4 __attribute__((ext_vector_type(4)));
-using NtCfg = Cfg<128, 128, kNtBK, 64, 64>;  // the 2 x 2 wave grid, for store_acc
-
-struct NtTile {
-    static constexpr int kPitch = KcTile<kNtBK>::kPitch;
-    static constexpr int kFloats = 128 * kPitch;
-    static constexpr int kLoads = 128 * kNtBK / 4 / 256;  // float4 per thread per operand
-    // float4 q of the tile (row q / 8, k 4 (q % 8)) of rows r0.. at k0.
-    __device__ __forceinline__ static void load(const float* p, int64_t ld, int64_t r0,
-                                                int64_t k0, nt4 (&r)[kLoads]) {
-#pragma unroll
-        for (int i = 0; i < kLoads; ++i) {
-            const int q = threadIdx.x + 256 * i;
-            r[i] = *reinterpret_cast<const nt4*>(p + (r0 + q / (kNtBK / 4)) * ld + k0 +
-                                                 4 * (q % (kNtBK / 4)));
-        }
-    }
-    __device__ __forceinline__ static void store(float* s, const nt4 (&r)[kLoads]) {
-#pragma unroll
-        for (int i = 0; i < kLoads; ++i) {
-            const int q = threadIdx.x + 256 * i;
-            *reinterpret_cast<nt4*>(s + (q / (kNtBK / 4)) * kPitch + 4 * (q % (kNtBK / 4))) = r[i];
-        }
-    }
-};
-
-template <bool EPI>
-__global__ __launch_bounds__(256) void gemm_nt_pipe(GemmArgs g) {
-    constexpr int kStage = 2 * NtTile::kFloats;
-    __shared__ __align__(16) float lds[2 * kStage];
-    const int tiles = g.tiles_m * g.tiles_n;
-    int bid = blockIdx.x;
-    if (tiles % 8 == 0) bid = (bid % 8) * (tiles / 8) + bid / 8;
-    constexpr int kGroupM = 8;
-    const int group = bid / (kGroupM * g.tiles_n);
-    const int first_m = group * kGroupM;
-    const int gsz = min(g.tiles_m - first_m, kGroupM);
-    const int in_group = bid % (kGroupM * g.tiles_n);
-    const int tm = first_m + in_group % gsz, tn = in_group / gsz;
-    const int64_t m0 = int64_t(tm) * 128, n0 = int64_t(tn) * 128;
-    const int split = blockIdx.y;
-    const int64_t k_begin = int64_t(split) * g.k_chunk;
-    const int64_t k_end = min(k_begin + g.k_chunk, g.k);
-    const int steps = __builtin_amdgcn_readfirstlane(int((k_end - k_begin) / kNtBK));
-    const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-    const int wm0 = (wave / 2) * 64, wn0 = (wave % 2) * 64;
-    constexpr int P = NtTile::kPitch;
-
-    floatx16 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-    nt4 ra[NtTile::kLoads], rb[NtTile::kLoads];
-    if (steps > 0) {
-        NtTile::load(g.a, g.lda, m0, k_begin, ra);
-        NtTile::load(g.b, g.ldb, n0, k_begin, rb);
-        NtTile::store(lds, ra);
-        NtTile::store(lds + NtTile::kFloats, rb);
-        if (steps > 1) {
-            NtTile::load(g.a, g.lda, m0, k_begin + kNtBK, ra);
-            NtTile::load(g.b, g.ldb, n0, k_begin + kNtBK, rb);
-        }
-        __syncthreads();
-    }
-    for (int s = 0; s < steps; ++s) {
-        const float* sa = lds + (s & 1) * kStage;
-        const float* sb = sa + NtTile::kFloats;
-        const float* pa = sa + (wm0 + lane % 32) * P + 4 * (lane / 32);
-        const float* pb = sb + (wn0 + lane % 32) * P + 4 * (lane / 32);
-        nt4 fa[2][2], fb[2][2];  // [register set][block]
-#pragma unroll
-        for (int i = 0; i < 2; ++i) fa[0][i] = *reinterpret_cast<const nt4*>(pa + 32 * i * P);
-#pragma unroll
-        for (int j = 0; j < 2; ++j) fb[0][j] = *reinterpret_cast<const nt4*>(pb + 32 * j * P);
-#pragma unroll
-        for (int kb = 0; kb < kNtBK; kb += 8) {
-            const int f = (kb / 8) & 1;
-            if (kb + 8 < kNtBK) {
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-                    fa[f ^ 1][i] = *reinterpret_cast<const nt4*>(pa + 32 * i * P + kb + 8);
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    fb[f ^ 1][j] = *reinterpret_cast<const nt4*>(pb + 32 * j * P + kb + 8);
-            }
-            if (kb == 8 && s + 1 < steps) {
-                // The other stage was last read before the previous barrier.
-                float* st = lds + ((s + 1) & 1) * kStage;
-                NtTile::store(st, ra);
-                NtTile::store(st + NtTile::kFloats, rb);
-                if (s + 2 < steps) {
-                    const int64_t kn = k_begin + int64_t(s + 2) * kNtBK;
-                    NtTile::load(g.a, g.lda, m0, kn, ra);
-                    NtTile::load(g.b, g.ldb, n0, kn, rb);
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[f][i][q], fb[f][j][q],
-                                                                         acc[i][j], 0, 0, 0);
-                    }
-        }
-        __syncthreads();
-    }
-    float* Cp = g.splits > 1 ? g.c + int64_t(split) * g.ws_stride : g.c;
-    const int64_t ldc = g.splits > 1 ? g.n : g.ldc;
-    store_acc<NtCfg, false, EPI>(g, acc, Cp, ldc, g.splits > 1 ? nullptr : g.add, m0, n0, wm0,
-                                 wn0, lane);
-}
-
 // ------------------------------------------------------------ K-sliced tiles
 //
 // Products whose output is too small to give every CU a 64 x 64 tile (512^3

@@ -1,0 +1,521 @@
+// gemm_split.hpp -- the staged-tile GEMM: fp32 products on the bf16 matrix instructions. Each
+// fp32 operand is the exact sum of three bf16 values, and the product is formed from six of the
+// nine products of the parts, accumulated in fp32.
+//
+// x = h + m + l, each the round-to-nearest bf16 of what is left: 24 significand bits in
+// 3 x 8, so the split is exact for |x| >= 2^-110. Of a b's nine part products the three
+// smallest (m l, l m, l l: at most 2^-25 of |a b| together) are dropped; the six others are
+// formed exactly by the matrix instruction and added to the fp32 accumulator.
+// v_mfma_f32_16x16x32_bf16 does 16 times the multiply-adds per cycle of the fp32 instructions,
+// so six of them cost 3/8 of the fp32 product's matrix time.
+//
+// Error, against 64-bit products of normal operands (2-norms): K = 64 9.2e-8, K = 1024 4.85e-7,
+// K = 4096 9.7e-7, where the chain of v_mfma_f32_32x32x2f32 that it replaces has 1.5e-7, 5.7e-7
+// and 1.1e-6: the accumulator is rounded 6 times per 32 k instead of 16. (All nine products
+// give the same figures.)
+//
+// What bounds it: the matrix pipe at the clock the chip sustains. The bare instruction reaches
+// 1,950 TFLOP/s of its 2,500, i.e. 325 fp32 TFLOP/s with six products; 8192 x 1024 x 4096 runs
+// 222-236 (fp32 instructions: 127-131), the conversion taking about a third of the issue slots
+// beside it. Measured and left out: the 32 x 32 x 16 instruction (212-227), the conversion
+// before or after the products by halves of the waves (200-207), raised priority around the
+// products (216-232), the products of a step summed apart and added to the accumulator once
+// per 32 k (error / 2.3, but 195-221).
+#ifndef EHIP_GEMM_SPLIT_HPP
+#define EHIP_GEMM_SPLIT_HPP
+
+#include "gemm_kernel.hpp"
+
+namespace ehip {
+namespace gemm_detail {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+// Four floats at any float's address (global memory takes 16-byte accesses at 4-byte
+// alignment on gfx950).
+typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
+// A byte address in global memory, said so: loads through an address whose origin the compiler
+// cannot see would otherwise be flat ones, which also occupy the LDS counter.
+typedef const __attribute__((address_space(1))) char* global_bytes;
+
+template <class T>
+__device__ __forceinline__ T global_load(global_bytes p) {
+    return *reinterpret_cast<const __attribute__((address_space(1))) T*>(p);
+}
+
+__device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2){a, b}, bf16x2));
+}
+
+// The three parts of a and b, two bf16 to a word. `bad` turns inf or NaN, and stays so, when
+// an operand is inf or NaN (or rounds to inf): its last remainder is then NaN.
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t& h, uint32_t& m,
+                                           uint32_t& l, float& bad) {
+    h = bf16_pair(a, b);
+    float ra = a - __builtin_bit_cast(float, h << 16);
+    float rb = b - __builtin_bit_cast(float, h & 0xffff0000u);
+    m = bf16_pair(ra, rb);
+    ra = ra - __builtin_bit_cast(float, m << 16);
+    rb = rb - __builtin_bit_cast(float, m & 0xffff0000u);
+    l = bf16_pair(ra, rb);
+    bad = __builtin_fmaf(ra, rb, bad);
+}
+
+constexpr int kSplitBK = 32;
+
+// One operand's tile of ROWS rows (of op(A), or columns of op(B)) by 32 k. KC: element (r, k)
+// is at p[r * ld + k], else at p[k * ld + r]. A thread stages kUnits units of one row by 8
+// consecutive k: loaded as two 16-byte loads (KC; four lanes read a row's 128 bytes) or as
+// eight 4-byte loads (a wave reads 256 consecutive bytes), either way ending in the eight
+// registers that pack into one 16-byte LDS write per part, with no transposition.
+//
+// LDS: three planes (h, m, l), each 16-row blocks of 1 KiB holding [k / 8][row % 16] 16-byte
+// groups, which is the matrix instruction's operand order: one conflict-free ds_read_b128 per
+// 16 x 32 block. The row's place is permuted within its group of 16 so that the writes of
+// eight lanes also fall on different banks, whether they hold two rows by four k groups (KC)
+// or eight rows.
+template <int ROWS, bool KC, int THREADS>
+struct SplitTile {
+    static constexpr int kUnits = ROWS * (kSplitBK / 8) / THREADS;
+    static constexpr int kPlane = ROWS * kSplitBK * 2;  // bytes
+    static_assert(kUnits >= 1 && kUnits * THREADS == ROWS * (kSplitBK / 8), "tile shape");
+
+    float v[kUnits][8];
+
+    __device__ __forceinline__ static int row(int u) {
+        const int q = int(threadIdx.x) + u * THREADS;
+        return KC ? q / 4 : q % ROWS;
+    }
+    __device__ __forceinline__ static int group(int u) {
+        const int q = int(threadIdx.x) + u * THREADS;
+        return KC ? q % 4 : q / ROWS;
+    }
+    __device__ __forceinline__ static int slot(int r, int kc) {
+        return (r / 16) * 1024 + kc * 256 + (((r & 15) ^ ((r >> 3) & 1) ^ (2 * kc)) << 4);
+    }
+    // Byte offsets of the thread's units from the tile's first element; rows past the last
+    // one repeat it (their results are not stored).
+    __device__ __forceinline__ static void offsets(uint32_t (&o)[kUnits], int64_t ld,
+                                                   int64_t rows_left) {
+#pragma unroll
+        for (int u = 0; u < kUnits; ++u) {
+            const int64_t r = row(u) < rows_left ? row(u) : rows_left - 1;
+            o[u] = uint32_t(4 * (KC ? r * ld + 8 * group(u) : 8 * group(u) * ld + r));
+        }
+    }
+    __device__ __forceinline__ void load(global_bytes base, const uint32_t (&o)[kUnits],
+                                         int64_t ld) {
+#pragma unroll
+        for (int u = 0; u < kUnits; ++u) {
+            if constexpr (KC) {
+                const floatx4u x = global_load<floatx4u>(base + o[u]);
+                const floatx4u y = global_load<floatx4u>(base + o[u] + 16);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    v[u][j] = x[j];
+                    v[u][4 + j] = y[j];
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    v[u][j] = global_load<float>(base + 4 * j * ld + o[u]);
+            }
+        }
+    }
+    // The same for a tile of which only the first `left` k are in the matrix (zeros after
+    // them), with 64-bit offsets: the last step of a K that is no multiple of 32, and every
+    // step where a leading dimension is too large for offsets().
+    __device__ __forceinline__ void load_tail(global_bytes base, int64_t ld, int64_t rows_left,
+                                              int left) {
+#pragma unroll
+        for (int u = 0; u < kUnits; ++u) {
+            const int64_t r = row(u) < rows_left ? row(u) : rows_left - 1;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int k = 8 * group(u) + j;
+                const int64_t kk = k < left ? k : 0;
+                const float x = global_load<float>(base + 4 * (KC ? r * ld + kk : kk * ld + r));
+                v[u][j] = k < left ? x : 0.0f;
+            }
+        }
+    }
+    __device__ __forceinline__ void store(char* lds, float& bad) const {
+#pragma unroll
+        for (int u = 0; u < kUnits; ++u) {
+            uintx4 h, m, l;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                uint32_t hj, mj, lj;
+                split_pair(v[u][2 * j], v[u][2 * j + 1], hj, mj, lj, bad);
+                h[j] = hj;
+                m[j] = mj;
+                l[j] = lj;
+            }
+            char* d = lds + slot(row(u), group(u));
+            *reinterpret_cast<uintx4*>(d) = h;
+            *reinterpret_cast<uintx4*>(d + kPlane) = m;
+            *reinterpret_cast<uintx4*>(d + 2 * kPlane) = l;
+        }
+    }
+};
+
+// Stores the wave's accumulators through the epilogue. Block (i, j), lane l, register r is
+// element (16 i + l % 16, 16 j + 4 (l / 16) + r) of the wave's tile: four consecutive columns
+// of a row per lane, one 16-byte access each for the output, the addend, the old output and
+// the residual. The loads of a block row come before its stores (the compiler cannot move a
+// load above an earlier store to C, which may alias it).
+template <int FM, int FN, bool CHECK, bool EPI>
+__device__ __forceinline__ void split_store(const GemmArgs& g, const floatx4 (&acc)[FM][FN],
+                                            float* Cp, int64_t ldc, const float* addp,
+                                            int64_t row0, int64_t col0) {
+    const auto get = [&](const float* p, int64_t col) {
+        if (!CHECK || col + 4 <= g.n) return floatx4(*reinterpret_cast<const floatx4u*>(p));
+        floatx4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (col + r < g.n) v[r] = p[r];
+        return v;
+    };
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+        const int64_t row = row0 + 16 * i;
+        if (CHECK && row >= g.m) continue;
+        floatx4 add[FN], old[FN], res[FN];
+        if constexpr (EPI) {
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                const int64_t col = col0 + 16 * j;
+                const floatx4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+                add[j] = old[j] = res[j] = zero;
+                if (CHECK && col >= g.n) continue;
+                if (addp != nullptr) {
+                    if (g.add_row) {
+                        const float a = addp[row];
+                        add[j] = (floatx4){a, a, a, a};
+                    } else {
+                        add[j] = get(addp + row * g.ld_add + col, col);
+                    }
+                }
+                if (g.beta != 0.0f) old[j] = get(Cp + row * ldc + col, col);
+                if (g.res != nullptr) res[j] = get(g.res + row * g.ld_res + col, col);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+            const int64_t col = col0 + 16 * j;
+            if (CHECK && col >= g.n) continue;
+            floatx4 v = acc[i][j];
+            if constexpr (EPI) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    v[r] = finish(g, v[r], add[j][r], old[j][r], res[j][r]);
+            }
+            float* dst = Cp + row * ldc + col;
+            if (!CHECK || col + 4 <= g.n) {
+                *reinterpret_cast<floatx4u*>(dst) = v;
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (col + r < g.n) dst[r] = v[r];
+            }
+        }
+    }
+}
+
+__device__ __forceinline__ int64_t uniform64(int64_t v) {
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(int(uint32_t(v)));
+    const uint32_t hi = __builtin_amdgcn_readfirstlane(int(uint32_t(uint64_t(v) >> 32)));
+    return int64_t(uint64_t(hi) << 32 | lo);
+}
+
+// Whether the byte offsets of SplitTile::offsets fit 32 bits (at most 256 rows of ld floats).
+__device__ __forceinline__ bool split_offsets_fit(const GemmArgs& g) {
+    return g.lda < (int64_t(1) << 21) && g.ldb < (int64_t(1) << 21);
+}
+
+template <int BM, int BN, int WM, int WN>
+struct TileThreads {
+    static constexpr int value = (BM / WM) * (BN / WN) * 64;
+};
+
+template <int BM, int BN, int WM, int WN, int STAGES, int MINW, bool TA, bool TB, bool COLSUM>
+__global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void gemm_kernel(
+    GemmArgs g) {
+    constexpr int kThreads = TileThreads<BM, BN, WM, WN>::value, kWaves = kThreads / 64;
+    using A = SplitTile<BM, !TA, kThreads>;
+    using B = SplitTile<BN, TB, kThreads>;
+    constexpr int kStage = 3 * (A::kPlane + B::kPlane);
+    constexpr int FM = WM / 16, FN = WN / 16;
+    __shared__ __attribute__((aligned(16))) char lds[STAGES * kStage];
+
+    const int tiles = g.tiles_m * g.tiles_n;
+    int tm, tn;
+    int64_t batch = g.batch0 + blockIdx.z;
+    if (g.causal != 0 && gridDim.y == 1) {
+        const int64_t lin = int64_t(blockIdx.z) * gridDim.x + blockIdx.x;
+        batch = g.batch0 + lin % gridDim.z;
+        const int t = int(lin / gridDim.z);
+        tm = t / g.tiles_n;
+        tn = t % g.tiles_n;
+    } else {
+        int bid = blockIdx.x;
+        if (tiles % 8 == 0) bid = (bid % 8) * (tiles / 8) + bid / 8;
+        constexpr int kGroupM = 8;
+        const int group = bid / (kGroupM * g.tiles_n);
+        const int first_m = group * kGroupM;
+        const int gsz = min(g.tiles_m - first_m, kGroupM);
+        const int in_group = bid % (kGroupM * g.tiles_n);
+        tm = first_m + in_group % gsz;
+        tn = in_group / gsz;
+    }
+    // Uniform by construction; said so, for the scalar addresses below (the divisions above
+    // run in vector registers).
+    tm = __builtin_amdgcn_readfirstlane(tm);
+    tn = __builtin_amdgcn_readfirstlane(tn);
+    batch = uniform64(batch);
+    const int split = blockIdx.y;
+    const float* Ap = g.a + uniform64(batch_offset(batch, g.inner, g.stride_a, g.stride_a2));
+    const float* Bp = g.b + uniform64(batch_offset(batch, g.inner, g.stride_b, g.stride_b2));
+    const int64_t m0 = int64_t(tm) * BM, n0 = int64_t(tn) * BN;
+    int64_t k_begin = int64_t(split) * g.k_chunk;
+    int64_t k_end = k_begin + g.k_chunk;
+    if (k_end > g.k) k_end = g.k;
+    if (g.causal == 4 && n0 >= m0 + BM) return;
+    if (g.causal == 1 && n0 >= m0 + BM) {
+        k_end = k_begin;
+    } else if (g.causal == 2) {
+        if (k_end > m0 + BM) k_end = k_begin > m0 + BM ? k_begin : m0 + BM;
+    } else if (g.causal == 3) {
+        if (k_begin < m0) k_begin = k_end < m0 ? k_end : m0;
+    }
+
+    const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+    const int wm0 = (wave / (BN / WN)) * WM, wn0 = (wave % (BN / WN)) * WN;
+
+    floatx4 acc[FM][FN];
+    const auto clear = [&]() {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[i][j] = (floatx4){0.0f, 0.0f, 0.0f, 0.0f};
+    };
+    clear();
+    const int steps =
+        __builtin_amdgcn_readfirstlane(int((k_end - k_begin + kSplitBK - 1) / kSplitBK));
+    // Whole steps, loaded without guards.
+    const int full = split_offsets_fit(g) ? int((k_end - k_begin) / kSplitBK) : 0;
+    const auto pa = (global_bytes)(TA ? Ap + k_begin * g.lda + m0 : Ap + m0 * g.lda + k_begin);
+    const auto pb = (global_bytes)(TB ? Bp + n0 * g.ldb + k_begin : Bp + k_begin * g.ldb + n0);
+    const int64_t da = 4 * kSplitBK * (TA ? g.lda : 1), db = 4 * kSplitBK * (TB ? 1 : g.ldb);
+    uint32_t oa[A::kUnits], ob[B::kUnits];
+    A::offsets(oa, g.lda, g.m - m0);
+    B::offsets(ob, g.ldb, g.n - n0);
+    A ta[2];
+    B tb[2];
+    float bad = 0.0f, csum[COLSUM ? B::kUnits : 1] = {};
+    const int fbase = A::slot(lane % 16, lane / 16);
+
+    // The step's base addresses, opaque to the optimiser: it would otherwise carry every
+    // load's address through the loop as a 64-bit register pair of its own (91 spilled
+    // registers in the A^T B form) instead of a scalar base and a 32-bit offset.
+    const auto scalar = [](global_bytes p) {
+        asm volatile("" : "+s"(p));
+        return p;
+    };
+    const auto load = [&](int s, int set) {
+        ta[set].load(TA ? scalar(pa + s * da) : pa + s * da, oa, g.lda);
+        tb[set].load(TB ? pb + s * db : scalar(pb + s * db), ob, g.ldb);
+    };
+    const auto load_any = [&](int s, int set) {
+        if (s < full) {
+            load(s, set);
+        } else {
+            const int left = int(min(k_end - k_begin - int64_t(s) * kSplitBK, int64_t(kSplitBK)));
+            ta[set].load_tail(pa + s * da, g.lda, g.m - m0, left);
+            tb[set].load_tail(pb + s * db, g.ldb, g.n - n0, left);
+        }
+    };
+    const auto convert = [&](int s, int set) {
+        char* st = lds + (STAGES == 2 ? (s & 1) * kStage : 0);
+        ta[set].store(st, bad);
+        tb[set].store(st + 3 * A::kPlane, bad);
+        if constexpr (COLSUM) {
+#pragma unroll
+            for (int u = 0; u < B::kUnits; ++u) {
+                const float* v = tb[set].v[u];
+                csum[u] += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+            }
+        }
+    };
+    const auto multiply = [&](int s) {
+        const char* st = lds + (STAGES == 2 ? (s & 1) * kStage : 0);
+        const char* sa = st + (wm0 / 16) * 1024 + fbase;
+        const char* sb = st + 3 * A::kPlane + (wn0 / 16) * 1024 + fbase;
+        // One block row of A at a time (all of them at once spill in the shapes that run three
+        // and four waves per SIMD). Smallest part products first; the operands swapped, so
+        // that a lane's four results are four consecutive columns of a row.
+        constexpr int kPart[6][2] = {{2, 0}, {1, 1}, {0, 2}, {1, 0}, {0, 1}, {0, 0}};
+        bf16x8 fb[3][FN];
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+            bf16x8 fa[3];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                fa[2 - q] =
+                    *reinterpret_cast<const bf16x8*>(sa + (2 - q) * A::kPlane + 1024 * i);
+                if (i == 0) {
+#pragma unroll
+                    for (int j = 0; j < FN; ++j)
+                        fb[q][j] = *reinterpret_cast<const bf16x8*>(sb + q * B::kPlane + 1024 * j);
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 6; ++q)
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        fb[kPart[q][1]][j], fa[kPart[q][0]], acc[i][j], 0, 0, 0);
+        }
+    };
+
+    if constexpr (STAGES == 2) {
+        if (steps > 0) {
+            load_any(0, 0);
+            if (steps > 1) load_any(1, 1);
+            convert(0, 0);
+            __syncthreads();
+        }
+        int s = 0;
+        for (; s + 3 < full; s += 2) {
+            load(s + 2, 0);
+            multiply(s);
+            convert(s + 1, 1);
+            __syncthreads();
+            load(s + 3, 1);
+            multiply(s + 1);
+            convert(s + 2, 0);
+            __syncthreads();
+        }
+        const auto last = [&](int t, int set) {
+            if (t + 2 < steps) load_any(t + 2, set ^ 1);
+            multiply(t);
+            if (t + 1 < steps) convert(t + 1, set);
+            __syncthreads();
+        };
+        for (; s < steps; s += 2) {
+            last(s, 1);
+            if (s + 1 < steps) last(s + 1, 0);
+        }
+    } else {
+        if (steps > 0) load_any(0, 0);
+        int s = 0;
+        for (; s + 1 < full; ++s) {
+            convert(s, 0);
+            load(s + 1, 0);
+            __syncthreads();
+            multiply(s);
+            __syncthreads();
+        }
+        for (; s < steps; ++s) {
+            convert(s, 0);
+            if (s + 1 < steps) load_any(s + 1, 0);
+            __syncthreads();
+            multiply(s);
+            __syncthreads();
+        }
+    }
+
+    // Operands the split cannot carry: inf and NaN (their parts would make NaN of results
+    // that are inf), and tiles of products so small that the parts fell below bf16's range.
+    // The tile is formed again by the fp32 instructions.
+    float big = 0.0f;
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) big = fmaxf(big, fabsf(acc[i][j][r]));
+    int flags = !(fabsf(bad) < __builtin_inff()) ? 1 : 0;
+    if (big > 0.0f) flags |= big < 0x1p-90f ? 2 : 4;
+    int* vote = reinterpret_cast<int*>(lds);
+    flags = (__any(flags & 1) ? 1 : 0) | (__any(flags & 2) ? 2 : 0) | (__any(flags & 4) ? 4 : 0);
+    if (lane == 0) vote[wave] = flags;
+    __syncthreads();
+    int all = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) all |= vote[w];
+    all = __builtin_amdgcn_readfirstlane(all);
+    if ((all & 1) || (all & 6) == 2) {
+        clear();
+#pragma unroll 1
+        for (int64_t k = k_begin; k < k_end; k += 4) {
+            const int64_t kk = k + lane / 16;
+            const bool in = kk < k_end;
+            float fa[FM], fb[FN];
+#pragma unroll
+            for (int i = 0; i < FM; ++i) {
+                const int64_t r = m0 + wm0 + 16 * i + lane % 16;
+                fa[i] = in && r < g.m ? (TA ? Ap[kk * g.lda + r] : Ap[r * g.lda + kk]) : 0.0f;
+            }
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                const int64_t c = n0 + wn0 + 16 * j + lane % 16;
+                fb[j] = in && c < g.n ? (TB ? Bp[c * g.ldb + kk] : Bp[kk * g.ldb + c]) : 0.0f;
+            }
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[j], fa[i], acc[i][j], 0, 0, 0);
+        }
+    }
+
+    if constexpr (COLSUM) {
+        // Column sums of B: a thread holds the sums over its k group of every step; the four
+        // groups of a column are added in order.
+        if (tm == 0) {
+            float* part = reinterpret_cast<float*>(lds) + 64;
+#pragma unroll
+            for (int u = 0; u < B::kUnits; ++u) part[B::group(u) * BN + B::row(u)] = csum[u];
+            __syncthreads();
+            const int c = threadIdx.x;
+            if (c < BN && n0 + c < g.n) {
+                const float v = ((part[c] + part[BN + c]) + part[2 * BN + c]) + part[3 * BN + c];
+                if (g.splits > 1)
+                    g.c[int64_t(split) * g.ws_stride + g.m * g.n + n0 + c] = v;
+                else
+                    g.colsum[n0 + c] = v;
+            }
+        }
+    }
+
+    float* Cp;
+    int64_t ldc;
+    if (g.splits > 1) {
+        Cp = g.c + int64_t(split) * g.ws_stride + batch * g.m * g.n;
+        ldc = g.n;
+    } else {
+        Cp = g.c + batch_offset(batch, g.inner, g.stride_c, g.stride_c2);
+        ldc = g.ldc;
+    }
+    const float* addp = g.add ? g.add + (int64_t(batch) % g.add_period) * g.stride_add : nullptr;
+    const bool inside = m0 + BM <= g.m && n0 + BN <= g.n;
+    const bool epi = g.splits == 1 && !plain_epilogue(g);
+    const int64_t row0 = m0 + wm0 + lane % 16, col0 = n0 + wn0 + 4 * (lane / 16);
+    if (inside && !epi)
+        split_store<FM, FN, false, false>(g, acc, Cp, ldc, addp, row0, col0);
+    else if (inside)
+        split_store<FM, FN, false, true>(g, acc, Cp, ldc, addp, row0, col0);
+    else if (!epi)
+        split_store<FM, FN, true, false>(g, acc, Cp, ldc, addp, row0, col0);
+    else
+        split_store<FM, FN, true, true>(g, acc, Cp, ldc, addp, row0, col0);
+}
+
+}  // namespace gemm_detail
+}  // namespace ehip
+
+#endif  // EHIP_GEMM_SPLIT_HPP

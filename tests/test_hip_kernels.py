@@ -1160,3 +1160,95 @@ def test_nt_pipeline_matches_staged_tiles(hip, m, n, k, epi):
             c[:m] += res  # the separate add the epilogue replaces
         outs.append(host(c[:m]))
     exact(outs[0], outs[1], f"pipeline vs staged ({epi})")
+
+
+# Staged products at the edges of their tiles: sizes one off the 64-, 128- and 256-element tiles,
+# K of less than a step, of whole steps and of odd remainders, with and without K splits.
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("m,n,k", [(2048, 2049, 1), (1030, 2050, 33), (257, 1281, 300),
+                                   (129, 4095, 517), (1999, 777, 1531), (4097, 130, 2049),
+                                   (100, 257, 3000)])
+def test_staged_products_edges(hip, ta, tb, m, n, k):
+    """op(A) op(B) with operands that start 4 bytes past an aligned address, against fp64 within
+    the statistical fp32 bound; with alpha, a bias row, beta, a residual and ReLU in the epilogue
+    the result is the plain product's, finished in that order."""
+    import torch
+    from ehip import GemmEx
+    from _hip import gemm_stat_bound
+    print_case("staged edges", ta, tb, m, n, k)
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    fa = torch.randn(m * k + 1, device="cuda", generator=g)
+    fb = torch.randn(n * k + 1, device="cuda", generator=g)
+    a = fa[1:].view(k, m) if ta else fa[1:].view(m, k)
+    b = fb[1:].view(n, k) if tb else fb[1:].view(k, n)
+    got = hip.gemm(a, b, trans_a=ta, trans_b=tb)
+    a64, b64 = a.double(), b.double()
+    a64, b64 = (a64.t() if ta else a64), (b64.t() if tb else b64)
+    bound = gemm_stat_bound(a64.norm(dim=1), b64.norm(dim=0), k) + 2.0 ** -22 * (a64 @ b64).abs()
+    err = (got.double() - a64 @ b64).abs()
+    assert bool((err <= bound).all()), float((err / bound).max())
+    bias = torch.randn(n, device="cuda", generator=g)
+    res = torch.randn(m, n, device="cuda", generator=g)
+    c0 = torch.randn(m, n, device="cuda", generator=g)
+    c = c0.clone()
+    d = GemmEx(trans_a=int(ta), trans_b=int(tb), batch=1, inner=1, m=m, n=n, k=k, a=hip.p(a),
+               lda=a.shape[1], b=hip.p(b), ldb=b.shape[1], c=hip.p(c), ldc=n, alpha=0.5,
+               addend=hip.p(bias), addend_period=1, beta=0.25, relu=1, residual=hip.p(res),
+               ld_residual=n)
+    hip.gemm_ex(d)
+    want = torch.relu(got * 0.5 + bias + 0.25 * c0 + res)
+    exact(host(c), host(want), "epilogue")
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+def test_staged_products_nonfinite_and_tiny(hip, ta, tb):
+    """An infinity, a NaN or a value that rounds past the largest bf16 gives what fp32 products
+    give (inf where the sum is inf, NaN only where it is); operands near the bottom of the fp32
+    range keep the accuracy of operands near 1, in tiles of every shape."""
+    import torch
+    from _hip import gemm_stat_bound
+    for m, n, k in [(512, 384, 768), (2048, 2048, 96), (257, 1281, 300)]:
+        print_case("staged nonfinite", ta, tb, m, n, k)
+        g = torch.Generator(device="cuda").manual_seed(k)
+        a = torch.randn((k, m) if ta else (m, k), device="cuda", generator=g)
+        b = torch.randn((n, k) if tb else (k, n), device="cuda", generator=g)
+        A, B = (a.t() if ta else a), (b.t() if tb else b)  # views of the stored operands
+        for scale in (1.0, 2.0 ** -110, 2.0 ** -122):
+            x = (A * scale).t().contiguous() if ta else (A * scale).contiguous()
+            want = (A.double() * scale) @ B.double()
+            got = hip.gemm(x, b, trans_a=ta, trans_b=tb).double()
+            bound = scale * gemm_stat_bound(A.double().norm(dim=1), B.double().norm(dim=0), k)
+            bound = bound + 2.0 ** -22 * want.abs() + k * 2.0 ** -149
+            assert bool(((got - want).abs() <= bound).all()), (m, n, k, scale)
+        clean = hip.gemm(a, b, trans_a=ta, trans_b=tb)
+        A[3, 5], A[m - 1, 7], A[10, 10] = float("inf"), float("nan"), 3.4e38
+        B[9, n - 3] = -float("inf")
+        got = host(hip.gemm(a, b, trans_a=ta, trans_b=tb))
+        want = host(A.double() @ B.double())
+        nan, inf = np.isnan(want), np.isinf(want)
+        assert np.array_equal(np.isnan(got), nan), (m, n, k)
+        assert np.array_equal(got[inf], want[inf].astype(np.float32)), (m, n, k)
+        rows = np.ones(m, bool)
+        rows[[3, 10, m - 1]] = False
+        cols = np.ones(n, bool)
+        cols[n - 3] = False
+        diff = np.abs(got - host(clean))[rows][:, cols]
+        assert diff.max() <= 1e-4, diff.max()  # the same sums by another instruction
+
+
+def test_staged_product_of_very_long_rows(hip):
+    """Leading dimensions past the 32-bit load offsets (rows of 2^21 floats)."""
+    import torch
+    from _hip import gemm_stat_bound
+    print_case("staged long rows")
+    ld, m, n, k = 1 << 21, 130, 70, 330
+    g = torch.Generator(device="cuda").manual_seed(9)
+    a = torch.empty(m, ld, device="cuda")
+    a[:, :k] = torch.randn(m, k, device="cuda", generator=g)
+    b = torch.randn(k, n, device="cuda", generator=g)
+    c = hip.f32((m, n))
+    hip.ok(hip.lib.ehip_gemm_f32(0, 0, 1, m, n, k, hip.p(a), ld, 0, hip.p(b), n, 0, 0.0, hip.p(c),
+                                 n, 0, hip.stream()), "gemm")
+    a64, b64 = a[:, :k].double(), b.double()
+    err = (c.double() - a64 @ b64).abs()
+    assert bool((err <= gemm_stat_bound(a64.norm(dim=1), b64.norm(dim=0), k)).all())
