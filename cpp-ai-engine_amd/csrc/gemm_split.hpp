@@ -162,6 +162,68 @@ struct SplitTile {
     }
 };
 
+// One staged K step of a wave: acc += its 16 FM x 16 FN tile over 32 k; sa and sb are the lane's
+// place in the first block of the operands' h planes. One block row of A at a time (all of them
+// at once spill in the shapes that run three and four waves per SIMD). Smallest part products
+// first; the operands swapped, so that a lane's four results are four consecutive columns of a
+// row.
+template <int FM, int FN, int PLANE_A, int PLANE_B>
+__device__ __forceinline__ void split_products(floatx4 (&acc)[FM][FN], const char* sa,
+                                               const char* sb) {
+    constexpr int kPart[6][2] = {{2, 0}, {1, 1}, {0, 2}, {1, 0}, {0, 1}, {0, 0}};
+    bf16x8 fb[3][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+        bf16x8 fa[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            fa[2 - q] = *reinterpret_cast<const bf16x8*>(sa + (2 - q) * PLANE_A + 1024 * i);
+            if (i == 0) {
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+                    fb[q][j] = *reinterpret_cast<const bf16x8*>(sb + q * PLANE_B + 1024 * j);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 6; ++q)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    fb[kPart[q][1]][j], fa[kPart[q][0]], acc[i][j], 0, 0, 0);
+    }
+}
+
+// Whether the workgroup's tile holds what the split cannot carry: inf or NaN among its operands
+// or results (the parts would make NaN of results that are inf, a product past the fp32 range
+// among them), or only results so small that parts fell below bf16's range. The tile is then formed again by the fp32 instructions. Every wave must
+// have finished reading the staged tiles (`lds`).
+template <int WAVES, int FM, int FN>
+__device__ __forceinline__ bool split_failed(const floatx4 (&acc)[FM][FN], float bad, char* lds) {
+    float big = 0.0f;
+    bool finite = fabsf(bad) < __builtin_inff();
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float v = fabsf(acc[i][j][r]);
+                finite = finite && v < __builtin_inff();
+                big = fmaxf(big, v);
+            }
+    int flags = finite ? 0 : 1;
+    if (big > 0.0f) flags |= big < 0x1p-90f ? 2 : 4;
+    int* vote = reinterpret_cast<int*>(lds);
+    flags = (__any(flags & 1) ? 1 : 0) | (__any(flags & 2) ? 2 : 0) | (__any(flags & 4) ? 4 : 0);
+    if (threadIdx.x % 64 == 0) vote[threadIdx.x / 64] = flags;
+    __syncthreads();
+    int all = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) all |= vote[w];
+    all = __builtin_amdgcn_readfirstlane(all);
+    return (all & 1) || (all & 6) == 2;
+}
+
 // Stores the wave's accumulators through the epilogue. Block (i, j), lane l, register r is
 // element (16 i + l % 16, 16 j + 4 (l / 16) + r) of the wave's tile: four consecutive columns
 // of a row per lane, one 16-byte access each for the output, the addend, the old output and
@@ -352,33 +414,9 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
     };
     const auto multiply = [&](int s) {
         const char* st = lds + (STAGES == 2 ? (s & 1) * kStage : 0);
-        const char* sa = st + (wm0 / 16) * 1024 + fbase;
-        const char* sb = st + 3 * A::kPlane + (wn0 / 16) * 1024 + fbase;
-        // One block row of A at a time (all of them at once spill in the shapes that run three
-        // and four waves per SIMD). Smallest part products first; the operands swapped, so
-        // that a lane's four results are four consecutive columns of a row.
-        constexpr int kPart[6][2] = {{2, 0}, {1, 1}, {0, 2}, {1, 0}, {0, 1}, {0, 0}};
-        bf16x8 fb[3][FN];
-#pragma unroll
-        for (int i = 0; i < FM; ++i) {
-            bf16x8 fa[3];
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                fa[2 - q] =
-                    *reinterpret_cast<const bf16x8*>(sa + (2 - q) * A::kPlane + 1024 * i);
-                if (i == 0) {
-#pragma unroll
-                    for (int j = 0; j < FN; ++j)
-                        fb[q][j] = *reinterpret_cast<const bf16x8*>(sb + q * B::kPlane + 1024 * j);
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < 6; ++q)
-#pragma unroll
-                for (int j = 0; j < FN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        fb[kPart[q][1]][j], fa[kPart[q][0]], acc[i][j], 0, 0, 0);
-        }
+        split_products<FM, FN, A::kPlane, B::kPlane>(
+            acc, st + (wm0 / 16) * 1024 + fbase,
+            st + 3 * A::kPlane + (wn0 / 16) * 1024 + fbase);
     };
 
     if constexpr (STAGES == 2) {
@@ -428,27 +466,7 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
         }
     }
 
-    // Operands the split cannot carry: inf and NaN (their parts would make NaN of results
-    // that are inf), and tiles of products so small that the parts fell below bf16's range.
-    // The tile is formed again by the fp32 instructions.
-    float big = 0.0f;
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) big = fmaxf(big, fabsf(acc[i][j][r]));
-    int flags = !(fabsf(bad) < __builtin_inff()) ? 1 : 0;
-    if (big > 0.0f) flags |= big < 0x1p-90f ? 2 : 4;
-    int* vote = reinterpret_cast<int*>(lds);
-    flags = (__any(flags & 1) ? 1 : 0) | (__any(flags & 2) ? 2 : 0) | (__any(flags & 4) ? 4 : 0);
-    if (lane == 0) vote[wave] = flags;
-    __syncthreads();
-    int all = 0;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) all |= vote[w];
-    all = __builtin_amdgcn_readfirstlane(all);
-    if ((all & 1) || (all & 6) == 2) {
+    if (split_failed<kWaves>(acc, bad, lds)) {
         clear();
 #pragma unroll 1
         for (int64_t k = k_begin; k < k_end; k += 4) {

@@ -1223,15 +1223,17 @@ def test_staged_products_nonfinite_and_tiny(hip, ta, tb):
         clean = hip.gemm(a, b, trans_a=ta, trans_b=tb)
         A[3, 5], A[m - 1, 7], A[10, 10] = float("inf"), float("nan"), 3.4e38
         B[9, n - 3] = -float("inf")
+        A[12, 11], B[11, 5] = 3e38, -3e38  # their product alone is past the fp32 range
         got = host(hip.gemm(a, b, trans_a=ta, trans_b=tb))
         want = host(A.double() @ B.double())
         nan, inf = np.isnan(want), np.isinf(want)
         assert np.array_equal(np.isnan(got), nan), (m, n, k)
         assert np.array_equal(got[inf], want[inf].astype(np.float32)), (m, n, k)
         rows = np.ones(m, bool)
-        rows[[3, 10, m - 1]] = False
+        rows[[3, 10, 12, m - 1]] = False
         cols = np.ones(n, bool)
-        cols[n - 3] = False
+        cols[[5, n - 3]] = False
+        assert got[12, 5] == -np.inf
         diff = np.abs(got - host(clean))[rows][:, cols]
         assert diff.max() <= 1e-4, diff.max()  # the same sums by another instruction
 
@@ -1252,3 +1254,27 @@ def test_staged_product_of_very_long_rows(hip):
     a64, b64 = a[:, :k].double(), b.double()
     err = (c.double() - a64 @ b64).abs()
     assert bool((err <= gemm_stat_bound(a64.norm(dim=1), b64.norm(dim=0), k)).all())
+
+
+@pytest.mark.parametrize("rows,cols", [(5, 1), (4099, 2), (700, 3), (1023, 5), (33, 1023),
+                                       (9, 1025), (2050, 2047), (1031, 4097), (3, 8191),
+                                       (4100, 4099)])
+def test_cross_entropy_backward_layouts(hip, rows, cols):
+    """(p - onehot) * (grad / rows) bit for bit from rows shorter than a four-element vector to
+    rows longer than a block's run, starting 4 bytes past an aligned address; targets outside
+    the row subtract nothing."""
+    import torch
+    print_case("xent backward", rows, cols)
+    r = rng(rows + cols)
+    flat = dev(r.random(rows * cols + 1, dtype=np.float32))
+    probs = flat[1:].view(rows, cols)
+    t = r.integers(0, cols, rows).astype(np.int32)
+    t[0], t[-1] = cols - 1, 0
+    t[rows // 2] = cols + 1
+    t[rows // 3] = -1
+    grad = np.float32(0.37)
+    got = host(hip.cross_entropy_backward(probs, dev(t), dev(np.array([grad], np.float32))))
+    want = host(probs).copy()
+    ok = (t >= 0) & (t < cols)
+    want[np.flatnonzero(ok), t[ok]] -= np.float32(1.0)
+    exact(got, want * np.float32(grad / np.float32(rows)), "dx")
