@@ -170,46 +170,6 @@ struct Workspace {
 // The grid's z extent: products beyond it run as further launches.
 constexpr int64_t kGridZ = 65535;
 
-// The staged tiles' shapes (gemm_kernel). per_cu: how many of a shape's workgroups a CU holds
-// (LDS and registers); rate: the throughput of a full CU relative to the first shape's,
-// measured on MI355X at 8192 x 1024 x 4096 and 4096^3 (224, 199, 177 and 150 TFLOP/s).
-struct TileShape {
-    int bm, bn, per_cu;
-    double rate;
-};
-constexpr TileShape kShapes[] = {{256, 128, 1, 1.0}, {128, 128, 2, 0.9}, {128, 64, 3, 0.78},
-                                 {64, 64, 3, 0.6}};
-// What is left of a CU's rate when it holds c of a shape's per_cu workgroups: alone, a
-// workgroup has nothing to run in its load and conversion phases (1999 x 1531 x 777 in 192
-// workgroups of 128 x 128: 56 us, in 576 of a third of K each: 46 us).
-double share(int c, int per_cu) {
-    if (c >= per_cu) return 1.0;
-    return c == 1 ? (per_cu == 2 ? 0.65 : 0.5) : 0.8;
-}
-
-// The shape with the least estimated time for an m x n output in `copies` products and K
-// splits: whole rounds of the chip's 256 CUs, then the last one's workgroups spread over
-// them. Every shape forms an element by the same chain of instructions, so the choice does
-// not change a bit.
-int choose_shape(int64_t m, int64_t n, int64_t copies) {
-    int best = 0;
-    double best_t = 0.0;
-    for (int i = 0; i < int(sizeof(kShapes) / sizeof(kShapes[0])); ++i) {
-        const TileShape& t = kShapes[i];
-        const int64_t work = ceil_div(m, t.bm) * ceil_div(n, t.bn) * copies;
-        const int64_t slots = int64_t(256) * t.per_cu;
-        const double unit = double(t.bm) * t.bn / t.rate;
-        const int last = int(ceil_div(work % slots, 256));
-        double time = double(work / slots) * t.per_cu * unit;
-        if (last > 0) time += last * unit / share(last, t.per_cu);
-        if (i == 0 || time < best_t) {
-            best = i;
-            best_t = time;
-        }
-    }
-    return best;
-}
-
 template <int BM, int BN, int WM, int WN, int STAGES, int MINW, bool TA, bool TB>
 int launch_shape(const GemmArgs& g, const dim3& grid, hipStream_t s) {
     constexpr int kThreads = TileThreads<BM, BN, WM, WN>::value;
@@ -225,55 +185,50 @@ int launch_shape(const GemmArgs& g, const dim3& grid, hipStream_t s) {
     return EHIP_OK;
 }
 
-// A product as staged tiles. The K split is planned on bm x bn tiles of bk (the planner's
-// class), whatever shape then runs: its number fixes the order of the sums and the
-// workspace.
+// A product as staged tiles. The most K splits are planned on bm x bn tiles of bk (the
+// planner's class): when the tile grid cannot fill the chip ("fill" is 256 workgroups of the
+// largest class and two per CU of the smaller ones) and K is long, up to ~512 workgroups, each
+// at least 8 K steps long.
+int class_splits(int64_t m, int64_t n, int64_t k, int64_t batch, int bm, int bn, int bk) {
+    const int64_t tiles = ceil_div(m, bm) * ceil_div(n, bn) * batch;
+    const int64_t fill = bm * bn >= 256 * 256 ? 256 : 512;
+    if (tiles >= fill || k < 16 * bk) return 1;
+    const int64_t want = std::min({ceil_div(512, tiles), k / (8 * bk), int64_t(256)});
+    const int64_t chunk = ceil_div(ceil_div(k, want), bk) * bk;
+    return int(ceil_div(k, chunk));
+}
+
 template <bool TA, bool TB>
 int launch_staged(const GemmArgs& g0, int64_t batch, int bm, int bn, int bk, hipStream_t s,
                   const Workspace& wsp) {
     GemmArgs g = g0;
-    // Split K when the tile grid alone cannot fill the chip and K is long: aim for ~512
-    // workgroups, each at least 8 K steps long. "Fill" is 256 workgroups of the largest
-    // class and two per CU (512) of the smaller ones.
-    const int64_t class_tiles = ceil_div(g.m, bm) * ceil_div(g.n, bn) * batch;
-    const int64_t fill = bm * bn >= 256 * 256 ? 256 : 512;
-    int splits = 1;
-    if (class_tiles < fill && g.k >= 16 * bk) {
-        int64_t want = ceil_div(512, class_tiles);
-        const int64_t max_by_k = g.k / (8 * bk);
-        if (want > max_by_k) want = max_by_k;
-        if (want > 256) want = 256;
-        if (want > 1) splits = int(want);
-    }
-    g.k_chunk = ceil_div(ceil_div(g.k, splits), kSplitBK) * kSplitBK;
-    splits = int(ceil_div(g.k, g.k_chunk));
+    const int most = class_splits(g.m, g.n, g.k, batch, bm, bn, bk);
+    StagedPlan plan = plan_staged(g.m, g.n, g.k, batch, most);
+    // Causal products skip by row bands of the tile, so they take the class's rows; the splits
+    // are those of the product without skipping, and so are the bits. The products whose tiles
+    // above the diagonal are left out write little but C: 64 columns at a time (256 heads of
+    // 512 x 512 x 64: 68 -> 64 us).
+    if (g.causal != 0) plan.shape = bm == 64 ? 3 : bn == 64 || g.causal == 1 || g.causal == 4 ? 2 : 1;
+    const int shape = plan.shape;
+    g.k_chunk = ceil_div(ceil_div(g.k, plan.splits), kSplitBK) * kSplitBK;
+    const int splits = int(ceil_div(g.k, g.k_chunk));
     g.splits = splits;
     // Unstored tiles would leave their split-K partials unwritten for the
     // reduction to read: split products store them as mode 1 does.
     if (splits > 1 && g.causal == 4) g.causal = 1;
     float* out = g.c;
     g.ws_stride = batch * g.m * g.n + (g.colsum ? g.n : 0);
+    // The no-allocation entry point admits what its array holds of the class's plan.
+    const size_t split_bytes = size_t(g.ws_stride) * sizeof(float);
+    if (wsp.base != nullptr && most > 1 && most * split_bytes > wsp.cap_bytes)
+        return fail(EHIP_EINVAL,
+                    "gemm (no allocation): %d K-splits of %lld x %lld need %zu bytes of "
+                    "workspace, more than the fixed %zu",
+                    most, (long long)g.m, (long long)g.n, most * split_bytes, wsp.cap_bytes);
     if (splits > 1) {
-        const size_t bytes = size_t(splits) * size_t(g.ws_stride) * sizeof(float);
-        float* ws = nullptr;
-        if (wsp.base != nullptr) {
-            if (bytes > wsp.cap_bytes)
-                return fail(EHIP_EINVAL,
-                            "gemm (no allocation): %d K-splits of %lld x %lld need %zu bytes of "
-                            "workspace, more than the fixed %zu",
-                            splits, (long long)g.m, (long long)g.n, bytes, wsp.cap_bytes);
-            ws = wsp.base;
-        } else {
-            ws = static_cast<float*>(scratch(bytes));
-            if (ws == nullptr) return EHIP_ENOMEM;
-        }
-        g.c = ws;
+        g.c = wsp.base != nullptr ? wsp.base : static_cast<float*>(scratch(splits * split_bytes));
+        if (g.c == nullptr) return EHIP_ENOMEM;
     }
-    // Causal products skip by row bands of the tile: they keep the class's shape.
-    const int shape = g.causal == 0 ? choose_shape(g.m, g.n, batch * splits)
-                      : bm == 64    ? 3
-                      : bn == 64    ? 2
-                                    : 1;
     g.tiles_m = int(ceil_div(g.m, kShapes[shape].bm));
     g.tiles_n = int(ceil_div(g.n, kShapes[shape].bn));
     const int64_t tiles = int64_t(g.tiles_m) * g.tiles_n;
@@ -531,6 +486,19 @@ int operand_alignment(const GemmArgs& g) {
     return (a ? 1 : 0) | (b ? 2 : 0);
 }
 
+// Whether 32 x 32 tiles with K sliced over the waves beat staged tiles on an output too small
+// for 512 of the latter. In whole tiles of 32, up to about 1.2e9 multiply-adds (MI355X, us,
+// sliced : staged: 512^3 5.8 : 10.5, 768^3 17.0 : 17.7, 3392 x 192 x 1984 42.6 : 32.4); with
+// edges or unaligned rows they load operand by operand and win only where the staged tiles
+// would leave most of the chip idle (697 x 80 x 272, 22 tiles of 64 x 64: 7.1 : 10.0;
+// 47 x 2464 x 656, 39 tiles: 13.7 : 10.2; 2394 x 368 x 1808: 101 : 37). Causal products stay:
+// their skipping keeps the bits of the full product either way.
+bool kslice_wins(const GemmArgs& g, int64_t batch) {
+    if (operands_aligned(g) && g.m % 32 == 0 && g.n % 32 == 0 && g.k % 32 == 0)
+        return double(g.m) * double(g.n) * double(g.k) * double(batch) < 1.2e9;
+    return ceil_div(g.m, 64) * ceil_div(g.n, 64) * batch < 32;
+}
+
 Tile plan_tile(const GemmArgs& g, int64_t batch, bool ta, bool tb) {
     const int64_t tl = ceil_div(g.m, 256) * ceil_div(g.n, 256) * batch;
     const int64_t tm = ceil_div(g.m, 128) * ceil_div(g.n, 128) * batch;
@@ -552,7 +520,9 @@ Tile plan_tile(const GemmArgs& g, int64_t batch, bool ta, bool tb) {
         ceil_div(g.m, 16) * ceil_div(g.n, 16) <= 1024)
         return Tile::P;
     // A B column sum is computed only by the staged tiles.
-    if (g.colsum == nullptr && ceil_div(g.m, 32) * ceil_div(g.n, 32) * batch >= 64) return Tile::K;
+    if (g.colsum == nullptr && ceil_div(g.m, 32) * ceil_div(g.n, 32) * batch >= 64 &&
+        kslice_wins(g, batch))
+        return Tile::K;
     return Tile::T;
 }
 

@@ -9,18 +9,20 @@
 // v_mfma_f32_16x16x32_bf16 does 16 times the multiply-adds per cycle of the fp32 instructions,
 // so six of them cost 3/8 of the fp32 product's matrix time.
 //
-// Error, against 64-bit products of normal operands (2-norms): K = 64 9.2e-8, K = 1024 4.85e-7,
-// K = 4096 9.7e-7, where the chain of v_mfma_f32_32x32x2f32 that it replaces has 1.5e-7, 5.7e-7
-// and 1.1e-6: the accumulator is rounded 6 times per 32 k instead of 16. (All nine products
-// give the same figures.)
+// Error, against 64-bit products (2-norms; normal operands): K = 64 4.6e-8, K = 1024 1.13e-7,
+// K = 4096 2.1e-7, where the chain of v_mfma_f32_32x32x2f32 that it replaces has 1.4e-7, 5.7e-7
+// and 1.15e-6 (half-normal operands, half of them zero: 4.4e-8, 1.12e-7, 2.1e-7 against 1.0e-7,
+// 4.0e-7 and 8.1e-7); the mean over a column is off by 1.7e-9 of the results' rms, against 3e-9
+// to 6e-9. A step's 32 k are summed apart from the accumulator and by turns negated
+// (split_products, split_flip); all nine part products would give the same figures.
 //
 // What bounds it: the matrix pipe at the clock the chip sustains. The bare instruction reaches
 // 1,950 TFLOP/s of its 2,500, i.e. 325 fp32 TFLOP/s with six products; 8192 x 1024 x 4096 runs
-// 222-236 (fp32 instructions: 127-131), the conversion taking about a third of the issue slots
-// beside it. Measured and left out: the 32 x 32 x 16 instruction (212-227), the conversion
-// before or after the products by halves of the waves (200-207), raised priority around the
-// products (216-232), the products of a step summed apart and added to the accumulator once
-// per 32 k (error / 2.3, but 195-221).
+// 217-221 (fp32 instructions: 127-131), the conversion and the sums taking about half of the
+// issue slots beside it. Measured and left out: the 32 x 32 x 16 instruction (212-227 where this
+// one, without the sums apart, has 222-236), the conversion before or after the products by
+// halves of the waves (200-207), raised priority around the products (216-232), loads two steps
+// ahead in a second register set (spills with the sums apart: 203-215).
 #ifndef EHIP_GEMM_SPLIT_HPP
 #define EHIP_GEMM_SPLIT_HPP
 
@@ -50,10 +52,10 @@ __device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2){a, b}, bf16x2));
 }
 
-// The three parts of a and b, two bf16 to a word. `bad` turns inf or NaN, and stays so, when
-// an operand is inf or NaN (or rounds to inf): its last remainder is then NaN.
+// The three parts of a and b, two bf16 to a word. An operand that is inf or NaN (or rounds to
+// inf) leaves NaN in its last part, and so in every result it takes part in.
 __device__ __forceinline__ void split_pair(float a, float b, uint32_t& h, uint32_t& m,
-                                           uint32_t& l, float& bad) {
+                                           uint32_t& l) {
     h = bf16_pair(a, b);
     float ra = a - __builtin_bit_cast(float, h << 16);
     float rb = b - __builtin_bit_cast(float, h & 0xffff0000u);
@@ -61,7 +63,6 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t& h, uint32
     ra = ra - __builtin_bit_cast(float, m << 16);
     rb = rb - __builtin_bit_cast(float, m & 0xffff0000u);
     l = bf16_pair(ra, rb);
-    bad = __builtin_fmaf(ra, rb, bad);
 }
 
 constexpr int kSplitBK = 32;
@@ -142,14 +143,18 @@ struct SplitTile {
             }
         }
     }
-    __device__ __forceinline__ void store(char* lds, float& bad) const {
+    // Splits the registers into the three planes; `flip` (the sign bit or 0) negates them first.
+    __device__ __forceinline__ void store(char* lds, uint32_t flip = 0) const {
+        const auto at = [&](int u, int j) {
+            return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v[u][j]) ^ flip);
+        };
 #pragma unroll
         for (int u = 0; u < kUnits; ++u) {
             uintx4 h, m, l;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 uint32_t hj, mj, lj;
-                split_pair(v[u][2 * j], v[u][2 * j + 1], hj, mj, lj, bad);
+                split_pair(at(u, 2 * j), at(u, 2 * j + 1), hj, mj, lj);
                 h[j] = hj;
                 m[j] = mj;
                 l[j] = lj;
@@ -162,15 +167,24 @@ struct SplitTile {
     }
 };
 
-// One staged K step of a wave: acc += its 16 FM x 16 FN tile over 32 k; sa and sb are the lane's
-// place in the first block of the operands' h planes. One block row of A at a time (all of them
-// at once spill in the shapes that run three and four waves per SIMD). Smallest part products
-// first; the operands swapped, so that a lane's four results are four consecutive columns of a
-// row.
+// The sign bit in odd K steps. The matrix instruction drops the low bits of its sums towards
+// minus infinity, which leaves every result the same fraction of an ulp low (3.4e-8 of their
+// rms at K = 1024): odd steps stage B negated and are subtracted, and the two cancel.
+__device__ __forceinline__ uint32_t split_flip(int s) { return uint32_t(s) << 31; }
+
+// One staged K step (s) of a wave: acc += its 16 FM x 16 FN tile over 32 k; sa and sb are the
+// lane's place in the first block of the operands' h planes. One block row of A at a time (all
+// of them at once spill in the shapes that run three and four waves per SIMD). Smallest part
+// products first; the operands swapped, so that a lane's four results are four consecutive
+// columns of a row. The step's sum is formed apart and added to the accumulator once, which
+// rounds the accumulator once per 32 k instead of once per 8 k of each part product (K = 1024:
+// error 4.85e-7 -> 1.18e-7, for 3 to 6 % of the time).
 template <int FM, int FN, int PLANE_A, int PLANE_B>
 __device__ __forceinline__ void split_products(floatx4 (&acc)[FM][FN], const char* sa,
-                                               const char* sb) {
-    constexpr int kPart[6][2] = {{2, 0}, {1, 1}, {0, 2}, {1, 0}, {0, 1}, {0, 0}};
+                                               const char* sb, int s) {
+    const float sign = __builtin_bit_cast(float, 0x3f800000u ^ split_flip(s));
+    constexpr int kPart[6][2] = {{1, 1}, {2, 0}, {0, 2}, {0, 1}, {1, 0}, {0, 0}};
+    constexpr int SUMS = 2;
     bf16x8 fb[3][FN];
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
@@ -185,22 +199,32 @@ __device__ __forceinline__ void split_products(floatx4 (&acc)[FM][FN], const cha
             }
         }
 #pragma unroll
-        for (int q = 0; q < 6; ++q)
+        for (int j0 = 0; j0 < FN; j0 += SUMS) {
+            floatx4 t[SUMS];
 #pragma unroll
-            for (int j = 0; j < FN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    fb[kPart[q][1]][j], fa[kPart[q][0]], acc[i][j], 0, 0, 0);
+            for (int q = 0; q < 6; ++q)
+#pragma unroll
+                for (int j = 0; j < SUMS; ++j)
+                    t[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        fb[kPart[q][1]][j0 + j], fa[kPart[q][0]],
+                        q == 0 ? (floatx4){0.0f, 0.0f, 0.0f, 0.0f} : t[j], 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < SUMS; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    acc[i][j0 + j][r] = __builtin_fmaf(t[j][r], sign, acc[i][j0 + j][r]);
+        }
     }
 }
 
-// Whether the workgroup's tile holds what the split cannot carry: inf or NaN among its operands
-// or results (the parts would make NaN of results that are inf, a product past the fp32 range
-// among them), or only results so small that parts fell below bf16's range. The tile is then formed again by the fp32 instructions. Every wave must
+// Whether the workgroup's tile holds what the split cannot carry: results that are not finite
+// (an inf or NaN among the operands makes NaN of every result it takes part in, and a product
+// past the fp32 range may), or only results so small that parts fell below bf16's range. The tile is then formed again by the fp32 instructions. Every wave must
 // have finished reading the staged tiles (`lds`).
 template <int WAVES, int FM, int FN>
-__device__ __forceinline__ bool split_failed(const floatx4 (&acc)[FM][FN], float bad, char* lds) {
+__device__ __forceinline__ bool split_failed(const floatx4 (&acc)[FM][FN], char* lds) {
     float big = 0.0f;
-    bool finite = fabsf(bad) < __builtin_inff();
+    bool finite = true;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -375,9 +399,9 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
     uint32_t oa[A::kUnits], ob[B::kUnits];
     A::offsets(oa, g.lda, g.m - m0);
     B::offsets(ob, g.ldb, g.n - n0);
-    A ta[2];
-    B tb[2];
-    float bad = 0.0f, csum[COLSUM ? B::kUnits : 1] = {};
+    A ta;
+    B tb;
+    float csum[COLSUM ? B::kUnits : 1] = {};
     const int fbase = A::slot(lane % 16, lane / 16);
 
     // The step's base addresses, opaque to the optimiser: it would otherwise carry every
@@ -387,27 +411,27 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
         asm volatile("" : "+s"(p));
         return p;
     };
-    const auto load = [&](int s, int set) {
-        ta[set].load(TA ? scalar(pa + s * da) : pa + s * da, oa, g.lda);
-        tb[set].load(TB ? pb + s * db : scalar(pb + s * db), ob, g.ldb);
+    const auto load = [&](int s) {
+        ta.load(TA ? scalar(pa + s * da) : pa + s * da, oa, g.lda);
+        tb.load(TB ? pb + s * db : scalar(pb + s * db), ob, g.ldb);
     };
-    const auto load_any = [&](int s, int set) {
+    const auto load_any = [&](int s) {
         if (s < full) {
-            load(s, set);
+            load(s);
         } else {
             const int left = int(min(k_end - k_begin - int64_t(s) * kSplitBK, int64_t(kSplitBK)));
-            ta[set].load_tail(pa + s * da, g.lda, g.m - m0, left);
-            tb[set].load_tail(pb + s * db, g.ldb, g.n - n0, left);
+            ta.load_tail(pa + s * da, g.lda, g.m - m0, left);
+            tb.load_tail(pb + s * db, g.ldb, g.n - n0, left);
         }
     };
-    const auto convert = [&](int s, int set) {
+    const auto convert = [&](int s) {
         char* st = lds + (STAGES == 2 ? (s & 1) * kStage : 0);
-        ta[set].store(st, bad);
-        tb[set].store(st + 3 * A::kPlane, bad);
+        ta.store(st);
+        tb.store(st + 3 * A::kPlane, split_flip(s));
         if constexpr (COLSUM) {
 #pragma unroll
             for (int u = 0; u < B::kUnits; ++u) {
-                const float* v = tb[set].v[u];
+                const float* v = tb.v[u];
                 csum[u] += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
             }
         }
@@ -416,57 +440,52 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
         const char* st = lds + (STAGES == 2 ? (s & 1) * kStage : 0);
         split_products<FM, FN, A::kPlane, B::kPlane>(
             acc, st + (wm0 / 16) * 1024 + fbase,
-            st + 3 * A::kPlane + (wn0 / 16) * 1024 + fbase);
+            st + 3 * A::kPlane + (wn0 / 16) * 1024 + fbase, s);
     };
 
+    // Two stages: while a step's products run, the next step is converted into the other stage
+    // and the one after it loaded. One stage: the waves of the CU's other workgroups fill the
+    // conversion phase.
     if constexpr (STAGES == 2) {
         if (steps > 0) {
-            load_any(0, 0);
-            if (steps > 1) load_any(1, 1);
-            convert(0, 0);
+            load_any(0);
+            convert(0);
+            if (steps > 1) load_any(1);
             __syncthreads();
         }
         int s = 0;
-        for (; s + 3 < full; s += 2) {
-            load(s + 2, 0);
+        for (; s + 2 < full; ++s) {
             multiply(s);
-            convert(s + 1, 1);
-            __syncthreads();
-            load(s + 3, 1);
-            multiply(s + 1);
-            convert(s + 2, 0);
+            convert(s + 1);
+            load(s + 2);
             __syncthreads();
         }
-        const auto last = [&](int t, int set) {
-            if (t + 2 < steps) load_any(t + 2, set ^ 1);
-            multiply(t);
-            if (t + 1 < steps) convert(t + 1, set);
+        for (; s < steps; ++s) {
+            multiply(s);
+            if (s + 1 < steps) convert(s + 1);
+            if (s + 2 < steps) load_any(s + 2);
             __syncthreads();
-        };
-        for (; s < steps; s += 2) {
-            last(s, 1);
-            if (s + 1 < steps) last(s + 1, 0);
         }
     } else {
-        if (steps > 0) load_any(0, 0);
+        if (steps > 0) load_any(0);
         int s = 0;
         for (; s + 1 < full; ++s) {
-            convert(s, 0);
-            load(s + 1, 0);
+            convert(s);
+            load(s + 1);
             __syncthreads();
             multiply(s);
             __syncthreads();
         }
         for (; s < steps; ++s) {
-            convert(s, 0);
-            if (s + 1 < steps) load_any(s + 1, 0);
+            convert(s);
+            if (s + 1 < steps) load_any(s + 1);
             __syncthreads();
             multiply(s);
             __syncthreads();
         }
     }
 
-    if (split_failed<kWaves>(acc, bad, lds)) {
+    if (split_failed<kWaves>(acc, lds)) {
         clear();
 #pragma unroll 1
         for (int64_t k = k_begin; k < k_end; k += 4) {
@@ -531,6 +550,62 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
         split_store<FM, FN, true, false>(g, acc, Cp, ldc, addp, row0, col0);
     else
         split_store<FM, FN, true, true>(g, acc, Cp, ldc, addp, row0, col0);
+}
+
+// The staged tiles' shapes (gemm_kernel). per_cu: how many of a shape's workgroups a CU holds
+// (LDS and registers); rate: the throughput of a full CU relative to the first shape's,
+// measured on MI355X at 8192 x 1024 x 4096 (217-221, 197, 171 and 152 TFLOP/s).
+struct TileShape {
+    int bm, bn, per_cu;
+    double rate;
+};
+inline constexpr TileShape kShapes[] = {{256, 128, 1, 1.0}, {128, 128, 2, 0.9}, {128, 64, 3, 0.78},
+                                        {64, 64, 3, 0.67}};
+constexpr double kCuFlopPerUs = 0.85e6;  // the first shape's, 218 TFLOP/s on 256 CUs
+// What is left of a CU's rate when it holds c of a shape's per_cu workgroups: alone, a
+// workgroup has nothing to run in its load and conversion phases (1999 x 1531 x 777 in 192
+// workgroups of 128 x 128: 56 us, in 576 of a third of K each: 46 us).
+inline double share(int c, int per_cu) {
+    if (c >= per_cu) return 1.0;
+    return c == 1 ? (per_cu == 2 ? 0.65 : 0.5) : 0.8;
+}
+
+struct StagedPlan {
+    int shape, splits;
+};
+
+// The shape and K split of least estimated time for `batch` products m x n x k, among the shapes
+// from `first` on and at most max_splits splits: whole rounds of the chip's 256 CUs, then the
+// last one's workgroups spread over them, 3 us of prologue and epilogue per round; a split adds
+// its workspace traffic and the reduction (1999 x 1531 in 3 splits: 13 us, which one round of
+// 64 x 64 tiles over the whole K saves). No fewer than an eighth of max_splits: the chains of a
+// sum grow with fewer splits, and so does its error, with their length's square root -- these
+// tiles' is below a quarter of the error of the fp32 chains that max_splits was planned for.
+// Every shape forms an element by the same chain of instructions; the splits fix its bits.
+inline StagedPlan plan_staged(int64_t m, int64_t n, int64_t k, int64_t batch, int max_splits,
+                              int first = 0) {
+    StagedPlan best{first, max_splits};
+    double best_t = 0.0;
+    for (int s = (max_splits + 7) / 8; s <= max_splits; ++s) {
+        const int64_t chunk = ceil_div(ceil_div(k, s), kSplitBK) * kSplitBK;
+        if (s > 1 && ceil_div(k, chunk) != s) continue;
+        const double out = 4.0 * double(m) * double(n) * double(batch);
+        const double reduce = s > 1 ? 4.0 + out * (s + 1) / 4e6 + out * (s - 1) / 5e6 : 0.0;
+        for (int i = first; i < int(sizeof(kShapes) / sizeof(kShapes[0])); ++i) {
+            const TileShape& t = kShapes[i];
+            const int64_t work = ceil_div(m, t.bm) * ceil_div(n, t.bn) * batch * s;
+            const int64_t slots = int64_t(256) * t.per_cu;
+            const double unit = 2.0 * t.bm * t.bn * double(chunk) / (t.rate * kCuFlopPerUs);
+            const int last = int(ceil_div(work % slots, 256));
+            double time = reduce + double(work / slots) * (t.per_cu * unit + 3.0);
+            if (last > 0) time += last * unit / share(last, t.per_cu) + 3.0;
+            if (best_t == 0.0 || time < best_t) {
+                best = {i, s};
+                best_t = time;
+            }
+        }
+    }
+    return best;
 }
 
 }  // namespace gemm_detail
