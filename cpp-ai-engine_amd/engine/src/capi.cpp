@@ -73,11 +73,40 @@ void load_params(const std::vector<Tensor>& params, const float* flat) {
     }
 }
 
+// Reads the parameters into `flat`, in order. Those on the device are gathered there, up to
+// 256 MiB at a time, and come back in one download straight into `flat`: one wait instead of
+// one per tensor, and no host copy of each on the way (37 tensors, 1 MB: 1.0 -> 0.2 ms; 35
+// tensors, 103 MB: 17 -> 9 ms).
 void store_params(const std::vector<Tensor>& params, float* flat) {
+    constexpr size_t kGather = size_t(64) << 20;  // floats
     size_t off = 0;
-    for (const Tensor& p : params) {
-        std::memcpy(flat + off, p.data(), p.size() * sizeof(float));
-        off += p.size();
+    for (size_t i = 0; i < params.size();) {
+        size_t last = i, n = 0;
+        while (last < params.size() && params[last].storage().resident_on_device() &&
+               params[last].storage().size() == params[last].size() &&
+               (n == 0 || n + params[last].size() <= kGather))
+            n += params[last++].size();
+        if (n == 0) {
+            std::memcpy(flat + off, params[i].data(), params[i].size() * sizeof(float));
+            off += params[i++].size();
+            continue;
+        }
+        if (last == i + 1) {
+            engine::hip::check(ehip_memcpy_d2h(flat + off, params[i].storage().device(),
+                                               n * sizeof(float), nullptr),
+                               "parameter download");
+        } else {
+            engine::Storage gathered(n, 0.0f);
+            float* dst = gathered.device_write();
+            for (size_t j = i, at = 0; j < last; at += params[j++].size())
+                engine::hip::check(ehip_memcpy_d2d(dst + at, params[j].storage().device(),
+                                                   params[j].size() * sizeof(float), nullptr),
+                                   "parameter gather");
+            engine::hip::check(ehip_memcpy_d2h(flat + off, dst, n * sizeof(float), nullptr),
+                               "parameter download");
+        }
+        off += n;
+        i = last;
     }
 }
 
