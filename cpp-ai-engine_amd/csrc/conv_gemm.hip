@@ -1090,13 +1090,32 @@ int launch_product(GemmArgs g, int64_t batch, const ConvGeo& cg, bool vec_a, boo
     return EHIP_OK;
 }
 
-// As launch_product, on the split tiles: the K split is planned on the class's tiles.
+// 128 x 128 tiles for products of at least 128 x 128 that they cover with
+// little more padding than 64 x 64 tiles do, when they still make 256 or more
+// workgroups (with their K splits); 64 x 64 otherwise. Measured on MI355X
+// over ResNet-stage layers: the larger tile is up to 1.6x faster on 128- and
+// 256-channel layers, the smaller one up to 1.5x faster on 64-channel layers
+// and on short reductions over few tiles.
+bool large_tiles(int64_t m, int64_t n, int64_t batch, int64_t k) {
+    if (m < 128 || n < 128) return false;
+    const auto area = [&](int64_t t) {
+        return double(ceil_div(m, t) * t) * double(ceil_div(n, t) * t);
+    };
+    if (area(128) > 1.15 * area(64)) return false;
+    const int64_t blocks = ceil_div(m, 128) * ceil_div(n, 128) * batch;
+    return blocks * split_count(blocks, k, 32) >= 256;
+}
+
+// As launch_product, on the split tiles: the K split is planned on the class's tiles and on
+// the reduction k without the padding of g.k, so that no product is split (and takes the
+// shared scratch) that launch_product would not split.
 template <class Geo, template <int, int> class LA, template <int, int> class LB>
-int launch_split(GemmArgs g, int64_t batch, const Geo& cg, bool large, hipStream_t s) {
+int launch_split(GemmArgs g, int64_t batch, int64_t k, const Geo& cg, hipStream_t s) {
+    const bool large = large_tiles(g.m, g.n, batch, k);
     const int t = large ? 128 : 64;
     const StagedPlan plan = plan_staged(
         g.m, g.n, g.k, batch,
-        split_count(ceil_div(g.m, t) * ceil_div(g.n, t) * batch, g.k, large ? 32 : 16), 1);
+        split_count(ceil_div(g.m, t) * ceil_div(g.n, t) * batch, k, large ? 32 : 16), 1);
     const int shape = plan.shape;
     g.k_chunk = ceil_div(ceil_div(g.k, plan.splits), kSplitBK) * kSplitBK;
     const int splits = int(ceil_div(g.k, g.k_chunk));
@@ -1133,22 +1152,6 @@ int launch_split(GemmArgs g, int64_t batch, const Geo& cg, bool large, hipStream
 using Small = Cfg<64, 64, 16, 32, 32>;     // 4 waves of 32 x 32
 using Large = Cfg<128, 128, 32, 64, 32>;  // 8 waves of 64 x 32
 
-// 128 x 128 tiles for products of at least 128 x 128 that they cover with
-// little more padding than 64 x 64 tiles do, when they still make 256 or more
-// workgroups (with their K splits); 64 x 64 otherwise. Measured on MI355X
-// over ResNet-stage layers: the larger tile is up to 1.6x faster on 128- and
-// 256-channel layers, the smaller one up to 1.5x faster on 64-channel layers
-// and on short reductions over few tiles.
-bool large_tiles(int64_t m, int64_t n, int64_t batch, int64_t k) {
-    if (m < 128 || n < 128) return false;
-    const auto area = [&](int64_t t) {
-        return double(ceil_div(m, t) * t) * double(ceil_div(n, t) * t);
-    };
-    if (area(128) > 1.15 * area(64)) return false;
-    const int64_t blocks = ceil_div(m, 128) * ceil_div(n, 128) * batch;
-    return blocks * split_count(blocks, k, 32) >= 256;
-}
-
 template <template <class, int, int> class LA, template <class, int, int> class LB, bool EPI>
 int run_product(const GemmArgs& g, int64_t batch, const ConvGeo& cg, bool vec_a, bool vec_b,
                 hipStream_t s) {
@@ -1157,21 +1160,39 @@ int run_product(const GemmArgs& g, int64_t batch, const ConvGeo& cg, bool vec_a,
     return launch_product<Small, 16, LA, LB, EPI>(g, batch, cg, vec_a, vec_b, s);
 }
 
-// The tap-by-tap product (forward; dx with FLIP): repacks the weights into scratch slot 1,
-// then the split tiles. `g` carries m, n, c and the epilogue.
+// A call's own block for the packed weights (null: the product takes the gather kernels, which
+// need none). The library's scratch would be shared by calls that overlap on several streams or
+// threads. The arena's blocks are ordered with the null stream (or the calling thread's
+// capture), so only calls there take one; kPackFloats (64 MiB) holds 1024 x 1024 x 3 x 3 and
+// keeps what a call asks for beside its operands small.
+constexpr int64_t kPackFloats = int64_t(1) << 24;
+struct PackBlock {
+    void* p = nullptr;
+    PackBlock(void* stream, bool wanted, int64_t floats) {
+        if (wanted && stream == nullptr && floats <= kPackFloats &&
+            ehip_arena_alloc(size_t(floats) * sizeof(float), &p) != EHIP_OK)
+            p = nullptr;
+    }
+    ~PackBlock() { ehip_arena_free(p); }
+    PackBlock(const PackBlock&) = delete;
+    PackBlock& operator=(const PackBlock&) = delete;
+    float* data() const { return static_cast<float*>(p); }
+};
+
+// The tap-by-tap product (forward; dx with FLIP): repacks the weights, then the split tiles.
+// `g` carries m, n, c and the epilogue.
 template <bool FLIP>
-int run_taps(GemmArgs g, int64_t batch, TapGeo tg, const float* weight, hipStream_t s) {
+int run_taps(GemmArgs g, int64_t batch, TapGeo tg, const float* weight, float* packed,
+             hipStream_t s) {
     const int taps = tg.kh * tg.kw;
-    const int64_t total = g.m * taps * tg.channels;  // below 2^31 (check_taps)
-    float* packed = static_cast<float*>(scratch(size_t(total) * sizeof(float), 1));
-    if (packed == nullptr) return EHIP_ENOMEM;
+    const int64_t total = g.m * taps * tg.channels;  // at most kPackFloats
     EHIP_LAUNCH("conv_pack_weights", conv_pack_weights<FLIP>, dim3(unsigned(ceil_div(total, 256))),
                 dim3(256), 0, s, weight, packed, total, tg.channels, taps, fast_div(tg.channels),
                 fast_div(taps));
     tg.packed = packed;
     g.k = int64_t(taps) * tg.padded;
-    return launch_split<TapGeo, PackedRows, TapPixels>(
-        g, batch, tg, large_tiles(g.m, g.n, batch, int64_t(taps) * tg.channels), s);
+    return launch_split<TapGeo, PackedRows, TapPixels>(g, batch, int64_t(taps) * tg.channels, tg,
+                                                       s);
 }
 
 TapGeo finish_taps(TapGeo tg) {
@@ -1185,11 +1206,10 @@ TapGeo finish_taps(TapGeo tg) {
 // Whether dW runs on the split tiles: 32 images of x within 32-bit byte offsets.
 bool takes_runs(const ConvGeo& cg) { return cg.chw < (int64_t(1) << 25) - 1; }
 
-// Whether a product over `channels` channels and `rows` output rows runs tap by tap: little
-// padding of the channels, and 32-bit offsets in the packed weights and in an image.
-bool takes_taps(int64_t channels, int64_t rows, int64_t taps, int64_t image) {
-    return channels >= kTapChannels && rows * taps * channels <= 0x7fffffffLL &&
-           4 * image <= 0xffffffffLL;
+// Whether a product over `channels` channels may run tap by tap: little padding of the
+// channels, and 32-bit offsets in an image.
+bool takes_taps(int64_t channels, int64_t image) {
+    return channels >= kTapChannels && 4 * image <= 0xffffffffLL;
 }
 
 // The stride phases of dx (stride 2..4, N s^2 <= 65535 products); false
@@ -1293,7 +1313,8 @@ int ehip_conv2d_igemm_f32(const float* x, const float* weight, const float* bias
     g.add_row = 1;
     g.add_period = 1;
     const hipStream_t s = as_stream(stream);
-    if (takes_taps(cg.c, cg.co, cg.khw, cg.hw)) {
+    const PackBlock packed(stream, takes_taps(cg.c, cg.hw), int64_t(cg.co) * cg.k);
+    if (packed.p != nullptr) {
         TapGeo tg{};
         tg.channels = cg.c;
         tg.h = cg.h;
@@ -1305,7 +1326,7 @@ int ehip_conv2d_igemm_f32(const float* x, const float* weight, const float* bias
         tg.kh = cg.kh;
         tg.kw = cg.kw;
         tg.in = x;
-        return run_taps<false>(g, win->batch, finish_taps(tg), weight, s);
+        return run_taps<false>(g, win->batch, finish_taps(tg), weight, packed.data(), s);
     }
     const bool vec_w = cg.k % 4 == 0 && aligned16(weight);
     if (bias) return run_product<WeightRows, ColsByPixel, true>(g, win->batch, cg, vec_w, false, s);
@@ -1346,8 +1367,7 @@ int ehip_conv2d_igemm_backward_f32(const float* x, const float* weight, const fl
         g.alpha = 1.0f;
         g.add_period = 1;
         const int rc = takes_runs(cg)
-                           ? launch_split<ConvGeo, DoutRows, TapRows>(
-                                 g, 1, cg, large_tiles(g.m, g.n, 1, g.k), s)
+                           ? launch_split<ConvGeo, DoutRows, TapRows>(g, 1, g.k, cg, s)
                            : run_product<DoutByChannel, ColsByTap, false>(g, 1, cg, vec_dout, false, s);
         if (rc) return rc;
     }
@@ -1395,7 +1415,9 @@ int ehip_conv2d_igemm_backward_f32(const float* x, const float* weight, const fl
             if (int rc2 = ehip_gemm_ex_f32(&d, stream)) return rc2;
             return ehip_col2im_f32(dcols, dx, win, stream);
         }
-        if (cg.stride == 1 && takes_taps(cg.co, cg.c, cg.khw, cg.p)) {
+        const PackBlock packed(stream, cg.stride == 1 && takes_taps(cg.co, cg.p),
+                               int64_t(cg.co) * cg.k);
+        if (packed.p != nullptr) {
             // The input gradient of a stride-1 layer is a convolution of dOut with the taps
             // reversed and the padding kH - 1 - pad.
             TapGeo tg{};
@@ -1410,7 +1432,7 @@ int ehip_conv2d_igemm_backward_f32(const float* x, const float* weight, const fl
             tg.kh = cg.kh;
             tg.kw = cg.kw;
             tg.in = grad_out;
-            rc = run_taps<true>(g, n, finish_taps(tg), weight, s);
+            rc = run_taps<true>(g, n, finish_taps(tg), weight, packed.data(), s);
         } else if (cg.stride == 1)
             rc = run_product<WeightByInput, DoutByPixelS1, false>(g, n, cg, false, false, s);
         else if (!plan_phases(cg, n, &ps, &phases, &max_count))

@@ -203,3 +203,76 @@ def test_conv_igemm_empty_batch_and_errors(hip):
                                                       None, ctypes.byref(w1), 8, hip.stream()),
                "dx without weight")
     assert hip.launched() == before
+
+
+# The tap-by-tap kernels' edges: channels one below, at and above the 24 they start at, off and
+# above their 32-channel steps on either side; 1x1 and even kernels; padding above kernel - 1 (the
+# input gradient's padding is then negative); stride 2; images smaller and larger than a tile.
+@pytest.mark.parametrize("shape,co,k,stride,pad", [((2, 23, 9, 11), 40, 3, 1, 1),
+                                                   ((2, 24, 9, 11), 23, 3, 1, 0),
+                                                   ((3, 25, 13, 7), 33, 3, 2, 1),
+                                                   ((2, 33, 6, 5), 24, 2, 1, 3),
+                                                   ((1, 40, 5, 9), 70, 1, 1, 0),
+                                                   ((2, 65, 12, 14), 130, 5, 1, 2)])
+def test_conv_igemm_tap_edges(hip, shape, co, k, stride, pad):
+    """On the null stream (tap by tap from 24 channels on) and on a named one (the gather kernels,
+    which need no packed weights): both within the worst-case fp32 bound of the exact product, and
+    an infinite input reaches the same outputs."""
+    import torch
+    print_case("conv-igemm-taps", shape, co, k, stride, pad)
+    r = np.random.default_rng(sum(shape) + co + k)
+    x = randn(r, *shape)
+    w = randn(r, co, shape[1], k, k)
+    b = randn(r, co)
+    oh, ow = ((s + 2 * pad - k) // stride + 1 for s in shape[2:])
+    g = randn(r, shape[0], co, oh, ow)
+    ex = exact_products(x, w, b, g, stride, pad)
+    bad = x.copy()
+    bad[0, shape[1] - 1, 1, 2] = np.inf
+    X, W, B, G, BAD = dev(x), dev(w), dev(b), dev(g), dev(bad)
+    torch.cuda.synchronize()
+    reached = []
+    for s in (torch.cuda.default_stream(), torch.cuda.Stream()):
+        with torch.cuda.stream(s):
+            Y = hip.conv2d_igemm(X, W, B, stride, pad)
+            DX, DW, DB = hip.conv2d_igemm_backward(X, W, G, stride, pad)
+            YB = hip.conv2d_igemm(BAD, W, B, stride, pad)
+            torch.cuda.synchronize()
+        within(host(Y), ex[0], "forward")
+        within(host(DX), ex[1], "dx")
+        within(host(DW), ex[2], "dweight")
+        within(host(DB), ex[3], "dbias")
+        reached.append(host(YB))
+    exact(np.isfinite(reached[0]).astype(np.float32), np.isfinite(reached[1]).astype(np.float32),
+          "outputs of an infinite input")
+
+
+@pytest.mark.parametrize("kind", ["conv", "product"])
+def test_overlapping_streams_share_no_workspace(hip, kind):
+    """Unsplit convolutions, and products of the K-sliced sizes that run on staged tiles, on two
+    streams at once: each keeps the bits that it has alone."""
+    import torch
+    print_case("overlapping streams", kind)
+    r = np.random.default_rng(7)
+    if kind == "conv":
+        args = [(dev(randn(r, 64, 64, 28, 28)), dev(randn(r, 64, 64, 3, 3))) for _ in range(2)]
+        run = lambda a: hip.conv2d_igemm(a[0], a[1], None, 1, 1)
+    else:
+        args = [(dev(randn(r, 697, 1361)), dev(randn(r, 1361, 810))) for _ in range(2)]
+        run = lambda a: hip.gemm(*a)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+
+    def on(i):
+        with torch.cuda.stream(streams[i]):
+            return run(args[i])
+
+    alone = []
+    for i in range(2):
+        alone.append(on(i))
+        torch.cuda.synchronize()
+    outs = [[on(i) for i in range(2)] for _ in range(8)]
+    torch.cuda.synchronize()
+    for pair in outs:
+        for got, want in zip(pair, alone):
+            exact(host(got), host(want), "overlapping call")
