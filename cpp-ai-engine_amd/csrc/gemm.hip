@@ -200,9 +200,9 @@ int class_splits(int64_t m, int64_t n, int64_t k, int64_t batch, int bm, int bn,
 
 template <bool TA, bool TB>
 int launch_staged(const GemmArgs& g0, int64_t batch, int bm, int bn, int bk, hipStream_t s,
-                  const Workspace& wsp) {
+                  const Workspace& wsp, bool unsplit = false) {
     GemmArgs g = g0;
-    const int most = class_splits(g.m, g.n, g.k, batch, bm, bn, bk);
+    const int most = unsplit ? 1 : class_splits(g.m, g.n, g.k, batch, bm, bn, bk);
     StagedPlan plan = plan_staged(g.m, g.n, g.k, batch, most);
     // Causal products skip by row bands of the tile, so they take the class's rows; the splits
     // are those of the product without skipping, and so are the bits. The products whose tiles
@@ -320,12 +320,14 @@ int launch_kslice(GemmArgs g, int64_t batch, hipStream_t s) {
 //      64 x 64 tiles; launch_staged then picks the shape that runs
 //   K  32 x 32 per workgroup, K sliced over its waves: outputs too small for
 //      the larger tiles to fill the chip (512^3, the char-Transformer's layers)
+//   U  products of K's sizes that staged tiles do faster, K unsplit: like K's they
+//      use no workspace, which overlapping calls on several streams would share
 //   P   16 x 16 per workgroup of 16 waves, each wave a sixteenth of K: A^T B
 //       products of few tiles over a long K (weight gradients of narrow
 //       layers), one load round trip per 128 k of a wave, no workspace
 // A tile size is taken when its grid fills the 256 CUs (with split-K where K
 // is long) and the padding it adds to the output stays small.
-enum class Tile { L, M, S, K, T, P };
+enum class Tile { L, M, S, K, T, U, P };
 
 // ------------------------------------------------------------ panel products
 //
@@ -520,9 +522,8 @@ Tile plan_tile(const GemmArgs& g, int64_t batch, bool ta, bool tb) {
         ceil_div(g.m, 16) * ceil_div(g.n, 16) <= 1024)
         return Tile::P;
     // A B column sum is computed only by the staged tiles.
-    if (g.colsum == nullptr && ceil_div(g.m, 32) * ceil_div(g.n, 32) * batch >= 64 &&
-        kslice_wins(g, batch))
-        return Tile::K;
+    if (g.colsum == nullptr && ceil_div(g.m, 32) * ceil_div(g.n, 32) * batch >= 64)
+        return kslice_wins(g, batch) ? Tile::K : Tile::U;
     return Tile::T;
 }
 
@@ -567,6 +568,7 @@ int gemm_modes(GemmArgs g, int64_t batch, hipStream_t s, const Workspace& wsp) {
         case Tile::S: return launch_staged<TA, TB>(g, batch, 128, 64, 32, s, wsp);
         case Tile::K: return launch_kslice<TA, TB>(g, batch, s);
         case Tile::P: return launch_panel(g, s);
+        case Tile::U: return launch_staged<TA, TB>(g, batch, 64, 64, 16, s, wsp, true);
         default: return launch_staged<TA, TB>(g, batch, 64, 64, 16, s, wsp);
     }
 }
