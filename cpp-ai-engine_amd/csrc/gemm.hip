@@ -488,17 +488,29 @@ int operand_alignment(const GemmArgs& g) {
     return (a ? 1 : 0) | (b ? 2 : 0);
 }
 
-// Whether 32 x 32 tiles with K sliced over the waves beat staged tiles on an output too small
-// for 512 of the latter. In whole tiles of 32, up to about 1.2e9 multiply-adds (MI355X, us,
-// sliced : staged: 512^3 5.8 : 10.5, 768^3 17.0 : 17.7, 3392 x 192 x 1984 42.6 : 32.4); with
-// edges or unaligned rows they load operand by operand and win only where the staged tiles
-// would leave most of the chip idle (697 x 80 x 272, 22 tiles of 64 x 64: 7.1 : 10.0;
-// 47 x 2464 x 656, 39 tiles: 13.7 : 10.2; 2394 x 368 x 1808: 101 : 37). Causal products stay:
-// their skipping keeps the bits of the full product either way.
-bool kslice_wins(const GemmArgs& g, int64_t batch) {
-    if (operands_aligned(g) && g.m % 32 == 0 && g.n % 32 == 0 && g.k % 32 == 0)
+// Whether 32 x 32 tiles with K sliced over the waves beat staged tiles of unsplit K on an
+// output too small for 512 of the latter (MI355X, us, sliced : staged). In whole tiles of 32, up
+// to about 1.2e9 multiply-adds (512^3 5.8 : 10.5, 768^3 17.0 : 17.7, 3392 x 192 x 1984 42.6 :
+// 32.4). With edges, by how the sliced tiles fill the chip:
+//   - to one per CU they win at every K beyond two staged steps (A B 3337 x 21 x 3303 62 : 73,
+//     A^T B 700 x 300 x 801 14 : 22, A^T B^T 8000 x 21 x 530 12 : 18), except A B^T from
+//     unaligned rows, whose loads are by element along both k: there only up to 256 k (8000 x 21
+//     x 250 9.5 : 10.0, x 801 22.6 : 21.6) and on few tiles (2100 x 21 x 2031 45 : 48);
+//   - to 448 tiles, A^T B (rows of both operands contiguous: 11000 x 31 x 1021 25 : 28.5, but x
+//     97 8.2 : 7.2) and, of aligned rows, A^T B^T (800 x 516 x 152 8.0 : 8.7) and the others
+//     at short K (A B 552 x 472 x 152 7.2 : 8.6, x 1012 25.9 : 26.1);
+//   - beyond, none (900 x 700 x 2031: A B 98 : 49, A B^T 142 : 48).
+// Causal products keep the bits of the full product either way.
+bool kslice_wins(const GemmArgs& g, int64_t batch, bool ta, bool tb) {
+    const bool rows = operands_aligned(g);
+    if (rows && g.m % 32 == 0 && g.n % 32 == 0 && g.k % 32 == 0)
         return double(g.m) * double(g.n) * double(g.k) * double(batch) < 1.2e9;
-    return ceil_div(g.m, 64) * ceil_div(g.n, 64) * batch < 32;
+    const int64_t tiles = ceil_div(g.m, 32) * ceil_div(g.n, 32) * batch;
+    if (tiles > 448) return false;
+    if (!ta && rows) return tiles <= 256 || g.k <= (tb ? 256 : 512);
+    if (!ta && tb) return tiles < 100 ? g.k > 64 : tiles <= 256 && g.k > 96 && g.k <= 256;
+    if (tiles <= 256 || (ta && tb && rows)) return g.k > 64;
+    return ta && !tb && g.k > 160;
 }
 
 Tile plan_tile(const GemmArgs& g, int64_t batch, bool ta, bool tb) {
@@ -523,7 +535,7 @@ Tile plan_tile(const GemmArgs& g, int64_t batch, bool ta, bool tb) {
         return Tile::P;
     // A B column sum is computed only by the staged tiles.
     if (g.colsum == nullptr && ceil_div(g.m, 32) * ceil_div(g.n, 32) * batch >= 64)
-        return kslice_wins(g, batch) ? Tile::K : Tile::U;
+        return kslice_wins(g, batch, ta, tb) ? Tile::K : Tile::U;
     return Tile::T;
 }
 
