@@ -581,9 +581,13 @@ struct StagedPlan {
 // 64 x 64 tiles over the whole K saves). No fewer than an eighth of max_splits: the chains of a
 // sum grow with fewer splits, and so does its error, with their length's square root -- these
 // tiles' is below a quarter of the error of the fp32 chains that max_splits was planned for.
+// The largest tile runs one workgroup per CU, so nothing covers its first loads and its stores:
+// not below 128 k (A B^T 8192 x 2048 x 16: 27 us, in 128 x 128 tiles 21; x 64 27 : 25; x 128
+// 36 : 34, 6564 x 1024 x 128 19 : 19).
 // Every shape forms an element by the same chain of instructions; the splits fix its bits.
 inline StagedPlan plan_staged(int64_t m, int64_t n, int64_t k, int64_t batch, int max_splits,
                               int first = 0) {
+    constexpr int kCount = int(sizeof(kShapes) / sizeof(kShapes[0]));
     StagedPlan best{first, max_splits};
     double best_t = 0.0;
     for (int s = (max_splits + 7) / 8; s <= max_splits; ++s) {
@@ -591,7 +595,7 @@ inline StagedPlan plan_staged(int64_t m, int64_t n, int64_t k, int64_t batch, in
         if (s > 1 && ceil_div(k, chunk) != s) continue;
         const double out = 4.0 * double(m) * double(n) * double(batch);
         const double reduce = s > 1 ? 4.0 + out * (s + 1) / 4e6 + out * (s - 1) / 5e6 : 0.0;
-        for (int i = first; i < int(sizeof(kShapes) / sizeof(kShapes[0])); ++i) {
+        for (int i = chunk < 128 && first == 0 ? 1 : first; i < kCount; ++i) {
             const TileShape& t = kShapes[i];
             const int64_t work = ceil_div(m, t.bm) * ceil_div(n, t.bn) * batch * s;
             const int64_t slots = int64_t(256) * t.per_cu;
