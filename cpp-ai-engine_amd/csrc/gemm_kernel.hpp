@@ -102,49 +102,7 @@ struct Cfg {
     static_assert(BK % 4 == 0, "BK");
 };
 
-// Loads a BM x BK tile of op(A) into registers. TA: A is stored K x M.
-// CHECK: zero-fill outside the matrix and use scalar loads.
-template <class C, int BM, int BK, bool TRANS, bool CHECK>
-__device__ __forceinline__ void load_tile(const float* __restrict__ p, int64_t ld, int64_t rows,
-                                          int64_t kdim, int64_t r0, int64_t k0, float4* reg,
-                                          int loads, int total, bool vec) {
-#pragma unroll
-    for (int i = 0; i < loads; ++i) {
-        const int q = threadIdx.x + i * C::kThreads;
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (q < total) {
-            int64_t r, kk;
-            if (!TRANS) {  // stored rows x K, 4 consecutive k
-                r = r0 + q / (BK / 4);
-                kk = k0 + 4 * (q % (BK / 4));
-                const float* src = p + r * ld + kk;
-                if (!CHECK || (vec && r < rows && kk + 3 < kdim)) {
-                    v = *reinterpret_cast<const float4*>(src);
-                } else if (r < rows) {
-                    v.x = kk < kdim ? src[0] : 0.f;
-                    v.y = kk + 1 < kdim ? src[1] : 0.f;
-                    v.z = kk + 2 < kdim ? src[2] : 0.f;
-                    v.w = kk + 3 < kdim ? src[3] : 0.f;
-                }
-            } else {  // stored K x rows, 4 consecutive rows
-                kk = k0 + q / (BM / 4);
-                r = r0 + 4 * (q % (BM / 4));
-                const float* src = p + kk * ld + r;
-                if (!CHECK || (vec && kk < kdim && r + 3 < rows)) {
-                    v = *reinterpret_cast<const float4*>(src);
-                } else if (kk < kdim) {
-                    v.x = r < rows ? src[0] : 0.f;
-                    v.y = r + 1 < rows ? src[1] : 0.f;
-                    v.z = r + 2 < rows ? src[2] : 0.f;
-                    v.w = r + 3 < rows ? src[3] : 0.f;
-                }
-            }
-        }
-        reg[i] = v;
-    }
-}
-
-// Stores the registers of load_tile into an LDS buffer laid out [k][row].
+// Stores the registers of a loaded tile into an LDS buffer laid out [k][row].
 template <class C, int BM, int BK, int LDS, bool TRANS>
 __device__ __forceinline__ void store_tile(float* __restrict__ s, const float4* reg, int loads,
                                            int total) {

@@ -210,8 +210,12 @@ int ehip_memcpy_d2d(void* dst, const void* src, size_t bytes, void* stream);
  * when trans_a != 0; likewise op(B) is k x n. stride_* is the element distance
  * between batch matrices; 0 shares one matrix across the batch (the reference's
  * unbatched operand). beta == 0 overwrites C without reading it.
- * fp32 MFMA (v_mfma_f32_32x32x2f32) with LDS-staged tiles; deterministic (a
- * fixed summation order per shape), not bit-equal to the CPU's serial sums.
+ * Large products run on the bf16 matrix instructions with each fp32 operand in
+ * three bf16 parts (24 bits, exact) and fp32 accumulation, small ones on the
+ * fp32 instructions; either way the result is that of an fp32 product, its
+ * error against 64 bits no larger than the fp32 instructions' chain.
+ * Deterministic (a fixed summation order per shape), not bit-equal to the
+ * CPU's serial sums.
  * Replaces cuda::ops::matmul (include/engine/detail/cuda_ops.hpp:46-47); the
  * transposed modes replace the materialised transposes of the backward pass
  * (src/tensor_ops.cpp:570-585). */
@@ -576,7 +580,7 @@ int ehip_conv2d_backward_weight_f32(const float* x, const float* grad_out, float
                                     float* dbias, const ehip_window_t* w, int64_t out_channels,
                                     void* stream);
 
-/* Implicit-GEMM convolution for layers of any width, on the fp32 MFMA tiles:
+/* Implicit-GEMM convolution for layers of any width, on the MFMA tiles:
  * the products of the reference's wide composition -- im2col, the product with
  * the transposed weight, the bias add and the permute to (N, C_out, oH, oW)
  * (src/conv.cpp:280-338, im2col/col2im src/conv.cpp:61-217) -- with the column
@@ -590,7 +594,10 @@ int ehip_conv2d_backward_weight_f32(const float* x, const float* grad_out, float
  *     cols; dbias = sum of grad_out per channel. Each output may be NULL to
  *     skip it; the ones given are overwritten.
  * Fixed-order sums (K split into fixed chunks on small grids): deterministic,
- * within the K-term tolerance of the reference's serial loops. Layers with
+ * within the K-term tolerance of the reference's serial loops. Forward and
+ * stride-1 dx of 24 or more gathered channels repack the weights into a block
+ * of the arena when `stream` is NULL (calls on other streams gather without
+ * one; both are within the same tolerance, not the same bits). Layers with
  * more than 2^31 - 1 elements in one image's input, output or weight rows, or
  * more than 65535 images, are refused with EHIP_EINVAL;
  * ehip_conv2d_igemm_supported() says 1 for a layer inside those limits (a
