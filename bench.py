@@ -863,6 +863,10 @@ def main():
     log("bench: dominant kernel (cfg5 weight-gradient products)")
     roof = in_step_roofline(rec["dw_probe"], dominant_kernel(eng, timer, torch))
     cpu = None
+    if not args.no_cpu and not os.path.exists(
+            os.path.join(ROOT, "oracle", "_ref", "libref_engine.so")):
+        log("bench: the compiled reference is not here: no CPU baselines")
+        args.no_cpu = True
     if not args.no_cpu:
         log("bench: reference CPU baseline (cfg5 sample)")
         cpu = cpu_cfg5_baseline(args.cpu_sample_batch)
