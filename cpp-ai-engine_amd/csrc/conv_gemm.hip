@@ -17,9 +17,9 @@
 // col2im, as a gather). dx thus reduces over C_out kH kW in (co, i, j) order
 // instead of col2im's sum over windows.
 //
-// The tiles are the GEMM's (fp32 MFMA 32x32x2, two LDS buffers, the next K
-// step's loads issued before the current MFMAs); only the operand loads
-// differ. Each thread decomposes the rows it gathers (output pixel, input
+// The tiles are the GEMM's (fp32 operands in bf16 parts, or fp32 MFMA 32x32x2;
+// the next K step's loads issued before the current MFMAs); only the operand
+// loads differ. Each thread decomposes the rows it gathers (output pixel, input
 // pixel, kernel tap) once per tile; per K step it decomposes the one reduction
 // index it starts from with multiply-shift division by the layer's invariant
 // divisors and steps the rest. Dense runs (weight rows, gradient rows of one

@@ -1167,7 +1167,11 @@ def test_nt_pipeline_matches_staged_tiles(hip, m, n, k, epi):
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("m,n,k", [(2048, 2049, 1), (1030, 2050, 33), (257, 1281, 300),
                                    (129, 4095, 517), (1999, 777, 1531), (4097, 130, 2049),
-                                   (100, 257, 3000)])
+                                   (100, 257, 3000),
+                                   # either side of 256 and of 448 tiles of 32 x 32, and of 64 k:
+                                   # K sliced over the waves, or staged with K unsplit
+                                   (8192, 21, 65), (8193, 21, 64), (8193, 31, 801),
+                                   (14336, 31, 161), (14337, 31, 160)])
 def test_staged_products_edges(hip, ta, tb, m, n, k):
     """op(A) op(B) with operands that start 4 bytes past an aligned address, against fp64 within
     the statistical fp32 bound; with alpha, a bias row, beta, a residual and ReLU in the epilogue
