@@ -774,12 +774,12 @@ struct TapPixels : SplitTile<ROWS, false, THREADS> {
     }
     // Zeroes the pixels in the padding: here, not in next(), so that nothing waits for the
     // loads before the products they are to overlap.
-    __device__ __forceinline__ void store(char* lds, uint32_t flip) {
+    __device__ __forceinline__ void store(char* lds, float scale) {
 #pragma unroll
         for (int u = 0; u < T::kUnits; ++u)
 #pragma unroll
             for (int e = 0; e < 8; ++e) this->v[u][e] = in[u] ? this->v[u][e] : 0.0f;
-        T::store(lds, flip);
+        T::store(lds, scale);
     }
     __device__ float at(int r, int64_t k) const {
         const int t = int(k / g.padded), c = int(k - int64_t(t) * g.padded);
@@ -894,12 +894,12 @@ struct TapRows : SplitTile<ROWS, true, THREADS> {
         }
         kr += 32;
     }
-    __device__ __forceinline__ void store(char* lds, uint32_t flip) {
+    __device__ __forceinline__ void store(char* lds, float scale) {
 #pragma unroll
         for (int u = 0; u < T::kUnits; ++u)
 #pragma unroll
             for (int e = 0; e < 8; ++e) this->v[u][e] = (in[u] >> e) & 1u ? this->v[u][e] : 0.0f;
-        T::store(lds, flip);
+        T::store(lds, scale);
     }
     __device__ float at(int r, int64_t k) const {
         if (r0 + r >= g.k) return 0.0f;
@@ -949,8 +949,8 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void co
         b.next();
     }
     for (int s = 0; s < steps; ++s) {
-        a.store(lds);
-        b.store(lds + 3 * A::kPlane, split_flip(s));
+        a.store(lds, split_scale(0));
+        b.store(lds + 3 * A::kPlane, split_scale(s));
         if (s + 1 < steps) {
             a.next();
             b.next();

@@ -2,10 +2,12 @@
 // fp32 operand is the exact sum of three bf16 values, and the product is formed from six of the
 // nine products of the parts, accumulated in fp32.
 //
-// x = h + m + l, each the round-to-nearest bf16 of what is left: 24 significand bits in
-// 3 x 8, so the split is exact for |x| >= 2^-110. Of a b's nine part products the three
-// smallest (m l, l m, l l: at most 2^-25 of |a b| together) are dropped; the six others are
-// formed exactly by the matrix instruction and added to the fp32 accumulator.
+// 2^24 x = h + m + l, each the round-to-nearest bf16 of what is left: 24 significand bits in
+// 3 x 8. The last bit of an fp32 value is 2^-149 or more, so every part that is not zero is at
+// least 2^-125, a normal bf16, and the split is exact for every |x| < 2^104. Of a b's nine part
+// products the three smallest (m l, l m, l l: at most 2^-25 of |a b| together) are dropped; the
+// six others are formed exactly by the matrix instruction and summed in fp32, 2^48 times their
+// value. A part product below the fp32 range at that scale is below 2^-197 of the result's.
 // v_mfma_f32_16x16x32_bf16 does 16 times the multiply-adds per cycle of the fp32 instructions,
 // so six of them cost 3/8 of the fp32 product's matrix time.
 //
@@ -52,8 +54,8 @@ __device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2){a, b}, bf16x2));
 }
 
-// The three parts of a and b, two bf16 to a word. An operand that is inf or NaN (or rounds to
-// inf) leaves NaN in its last part, and so in every result it takes part in.
+// The three parts of a and b (scaled), two bf16 to a word. An operand that is inf or NaN (or
+// scales or rounds to inf) leaves NaN in its last part, and so in every result it takes part in.
 __device__ __forceinline__ void split_pair(float a, float b, uint32_t& h, uint32_t& m,
                                            uint32_t& l) {
     h = bf16_pair(a, b);
@@ -143,18 +145,15 @@ struct SplitTile {
             }
         }
     }
-    // Splits the registers into the three planes; `flip` (the sign bit or 0) negates them first.
-    __device__ __forceinline__ void store(char* lds, uint32_t flip = 0) const {
-        const auto at = [&](int u, int j) {
-            return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v[u][j]) ^ flip);
-        };
+    // Splits the registers, times `scale` (split_scale), into the three planes.
+    __device__ __forceinline__ void store(char* lds, float scale) const {
 #pragma unroll
         for (int u = 0; u < kUnits; ++u) {
             uintx4 h, m, l;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 uint32_t hj, mj, lj;
-                split_pair(at(u, 2 * j), at(u, 2 * j + 1), hj, mj, lj);
+                split_pair(v[u][2 * j] * scale, v[u][2 * j + 1] * scale, hj, mj, lj);
                 h[j] = hj;
                 m[j] = mj;
                 l[j] = lj;
@@ -172,6 +171,18 @@ struct SplitTile {
 // rms at K = 1024): odd steps stage B negated and are subtracted, and the two cancel.
 __device__ __forceinline__ uint32_t split_flip(int s) { return uint32_t(s) << 31; }
 
+// What an operand is multiplied by as it is split: 2^24, which keeps the parts of the smallest
+// values inside bf16's range (without it a part is lost from |x| < 2^-110 on: a row of 2^-122
+// among rows of 1 kept 13 bits) for about 1 % of the time (8192 x 1024 x 4096 with both its
+// backward products 1039 -> 1050 us). A takes split_scale(0), B split_scale(s).
+__device__ __forceinline__ float split_scale(int s) {
+    return __builtin_bit_cast(float, 0x4b800000u ^ split_flip(s));
+}
+// What a step's sum is multiplied by as it is added to the accumulator: 2^-48.
+__device__ __forceinline__ float split_unscale(int s) {
+    return __builtin_bit_cast(float, 0x27800000u ^ split_flip(s));
+}
+
 // One staged K step (s) of a wave: acc += its 16 FM x 16 FN tile over 32 k; sa and sb are the
 // lane's place in the first block of the operands' h planes. One block row of A at a time (all
 // of them at once spill in the shapes that run three and four waves per SIMD). Smallest part
@@ -182,7 +193,7 @@ __device__ __forceinline__ uint32_t split_flip(int s) { return uint32_t(s) << 31
 template <int FM, int FN, int PLANE_A, int PLANE_B>
 __device__ __forceinline__ void split_products(floatx4 (&acc)[FM][FN], const char* sa,
                                                const char* sb, int s) {
-    const float sign = __builtin_bit_cast(float, 0x3f800000u ^ split_flip(s));
+    const float unscale = split_unscale(s);
     constexpr int kPart[6][2] = {{1, 1}, {2, 0}, {0, 2}, {0, 1}, {1, 0}, {0, 0}};
     constexpr int SUMS = 2;
     bf16x8 fb[3][FN];
@@ -212,40 +223,34 @@ __device__ __forceinline__ void split_products(floatx4 (&acc)[FM][FN], const cha
             for (int j = 0; j < SUMS; ++j)
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    acc[i][j0 + j][r] = __builtin_fmaf(t[j][r], sign, acc[i][j0 + j][r]);
+                    acc[i][j0 + j][r] = __builtin_fmaf(t[j][r], unscale, acc[i][j0 + j][r]);
         }
     }
 }
 
-// Whether the workgroup's tile holds what the split cannot carry: results that are not finite
-// (an inf or NaN among the operands makes NaN of every result it takes part in, and a product
-// past the fp32 range may), or only results so small that parts fell below bf16's range. The tile is then formed again by the fp32 instructions. Every wave must
-// have finished reading the staged tiles (`lds`).
+// Whether the workgroup's tile holds what the split cannot carry: a result that is not finite.
+// An inf or NaN among the operands, or a value of 2^104 or more, makes NaN of every result it
+// takes part in; 32 k whose products sum to 2^80 or more leave the fp32 range at the sums' scale.
+// The whole tile is then formed again by the fp32 instructions. Every wave must have finished
+// reading the staged tiles (`lds`).
 template <int WAVES, int FM, int FN>
 __device__ __forceinline__ bool split_failed(const floatx4 (&acc)[FM][FN], char* lds) {
-    float big = 0.0f;
     bool finite = true;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float v = fabsf(acc[i][j][r]);
-                finite = finite && v < __builtin_inff();
-                big = fmaxf(big, v);
-            }
-    int flags = finite ? 0 : 1;
-    if (big > 0.0f) flags |= big < 0x1p-90f ? 2 : 4;
+            for (int r = 0; r < 4; ++r)
+                finite = finite && fabsf(acc[i][j][r]) < __builtin_inff();
     int* vote = reinterpret_cast<int*>(lds);
-    flags = (__any(flags & 1) ? 1 : 0) | (__any(flags & 2) ? 2 : 0) | (__any(flags & 4) ? 4 : 0);
-    if (threadIdx.x % 64 == 0) vote[threadIdx.x / 64] = flags;
+    const int failed = __any(!finite) ? 1 : 0;
+    if (threadIdx.x % 64 == 0) vote[threadIdx.x / 64] = failed;
     __syncthreads();
-    int all = 0;
+    int any = 0;
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) all |= vote[w];
-    all = __builtin_amdgcn_readfirstlane(all);
-    return (all & 1) || (all & 6) == 2;
+    for (int w = 0; w < WAVES; ++w) any |= vote[w];
+    return __builtin_amdgcn_readfirstlane(any) != 0;
 }
 
 // Stores the wave's accumulators through the epilogue. Block (i, j), lane l, register r is
@@ -426,8 +431,8 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
     };
     const auto convert = [&](int s) {
         char* st = lds + (STAGES == 2 ? (s & 1) * kStage : 0);
-        ta.store(st);
-        tb.store(st + 3 * A::kPlane, split_flip(s));
+        ta.store(st, split_scale(0));
+        tb.store(st + 3 * A::kPlane, split_scale(s));
         if constexpr (COLSUM) {
 #pragma unroll
             for (int u = 0; u < B::kUnits; ++u) {

@@ -211,9 +211,12 @@ int ehip_memcpy_d2d(void* dst, const void* src, size_t bytes, void* stream);
  * between batch matrices; 0 shares one matrix across the batch (the reference's
  * unbatched operand). beta == 0 overwrites C without reading it.
  * Large products run on the bf16 matrix instructions with each fp32 operand in
- * three bf16 parts (24 bits, exact) and fp32 accumulation, small ones on the
- * fp32 instructions; either way the result is that of an fp32 product, its
- * error against 64 bits no larger than the fp32 instructions' chain.
+ * three bf16 parts (24 bits, exact for normal and subnormal values) and fp32
+ * accumulation, small ones on the fp32 instructions; either way the result is
+ * that of an fp32 product, its error against 64 bits no larger than the fp32
+ * instructions' chain. A tile of C with a result that is not finite, an operand
+ * of 2^104 or more, or 32 consecutive products that sum to 2^80 or more is
+ * formed by the fp32 instructions as a whole (the same value, other last bits).
  * Deterministic (a fixed summation order per shape), not bit-equal to the
  * CPU's serial sums.
  * Replaces cuda::ops::matmul (include/engine/detail/cuda_ops.hpp:46-47); the
@@ -296,7 +299,7 @@ int ehip_gemm_f32_noalloc(int trans_a, int trans_b, int64_t batch, int64_t m, in
  *      consumer that never reads j > i: the causal softmax pair below.
  * Skipped products are exact zeros, so every result keeps its value (its bits,
  * but for the sign of a sum that is exactly zero) as long as the operands are
- * finite; 0 computes everything. Honoured by the staged MFMA tiles; the other
+ * finite (and none that is skipped 2^104 or more); 0 computes everything. Honoured by the staged MFMA tiles; the other
  * kernels compute everything. (No counterpart in the reference, which
  * computes and then masks: src/transformer.cpp:279-304.) */
 typedef struct {

@@ -276,3 +276,29 @@ def test_overlapping_streams_share_no_workspace(hip, kind):
     for pair in outs:
         for got, want in zip(pair, alone):
             exact(host(got), host(want), "overlapping call")
+
+
+@pytest.mark.parametrize("shape,co,k,stride,pad", [((2, 33, 10, 11), 40, 3, 1, 1),
+                                                   ((3, 64, 7, 9), 65, 1, 2, 0)])
+@pytest.mark.parametrize("ew,ex,eg", [(-124, 60, 90), (60, -124, 40), (100, 90, -125),
+                                      (90, 60, -120)])
+def test_conv_igemm_wide_ranges(hip, shape, co, k, stride, pad, ew, ex, eg):
+    """Weights, inputs and gradients far from 1 on either side, and one tiny channel among
+    ordinary ones, keep fp32's accuracy: within the worst-case fp32 bound of the exact product."""
+    print_case("conv-igemm-ranges", shape, co, k, stride, pad, ew, ex, eg)
+    r = np.random.default_rng(co + abs(ew))
+    x = randn(r, *shape) * np.float32(2.0 ** ex)
+    w = randn(r, co, shape[1], k, k) * np.float32(2.0 ** ew)
+    x[:, 3] *= np.float32(2.0 ** -20)
+    w[5] *= np.float32(2.0 ** -20)
+    oh, ow = ((s + 2 * pad - k) // stride + 1 for s in shape[2:])
+    g = randn(r, shape[0], co, oh, ow) * np.float32(2.0 ** eg)
+    want = exact_products(x, w, None, g, stride, pad)
+    got = [hip.conv2d_igemm(dev(x), dev(w), None, stride, pad)]
+    got += hip.conv2d_igemm_backward(dev(x), dev(w), dev(g), stride, pad)
+    terms = (shape[1] * k * k, co * k * k, shape[0] * oh * ow, shape[0] * oh * ow)
+    for t, (e, bound), n, what in zip(got, want, terms, ("forward", "dx", "dweight", "dbias")):
+        if np.abs(e).max() < 2.0 ** 127:
+            # a subnormal's last bit for each addition beside the bound
+            worst = float(np.max(np.abs(host(t).astype(np.float64) - e) / (bound + n * 2.0 ** -149)))
+            assert worst <= 1.0, (what, worst)

@@ -1242,6 +1242,46 @@ def test_staged_products_nonfinite_and_tiny(hip, ta, tb):
         assert diff.max() <= 1e-4, diff.max()  # the same sums by another instruction
 
 
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("m,n,k", [(2048, 2048, 96), (257, 1281, 300), (1030, 2050, 33)])
+def test_staged_products_of_wide_ranges(hip, ta, tb, m, n, k):
+    """Operands of any normal or subnormal size keep their 24 bits: tiny rows and columns among
+    ordinary ones, tiny operands times large ones, subnormals, and rows whose sums leave the
+    range of the scaled step sums (re-formed by the fp32 instructions). Every element within the
+    statistical fp32 bound of its own row and column, and a subnormal's last bit for each of the
+    K additions."""
+    import torch
+    from _hip import gemm_stat_bound
+    print_case("staged ranges", ta, tb, m, n, k)
+    g = torch.Generator(device="cuda").manual_seed(m + k)
+    A = torch.randn(m, k, device="cuda", generator=g)
+    B = torch.randn(k, n, device="cuda", generator=g)
+
+    def check(a, b, what):
+        a, b = a.contiguous(), b.contiguous()
+        x, y = (a.t().contiguous() if ta else a), (b.t().contiguous() if tb else b)
+        got = hip.gemm(x, y, trans_a=ta, trans_b=tb).double()
+        a64, b64 = a.double(), b.double()
+        want = a64 @ b64
+        bound = gemm_stat_bound(a64.norm(dim=1), b64.norm(dim=0), k)
+        bound = bound + 2.0 ** -22 * want.abs() + k * 2.0 ** -149
+        worst = float(((got - want).abs() / bound).max())
+        assert worst <= 1.0, (what, worst)
+
+    rows, cols = A.clone(), B.clone()
+    for i, e in enumerate((-100, -112, -118, -122, -126, -135, -147)):
+        rows[7 + 17 * i] *= 2.0 ** e
+        cols[:, 11 + 13 * i] *= 2.0 ** e
+    check(rows, B, "tiny rows")
+    check(A, cols, "tiny columns")
+    for ea, eb in ((-120, 40), (-124, 60), (-125, 100), (-140, 103), (60, -124), (103, -140)):
+        check(A * 2.0 ** ea, B * 2.0 ** eb, (ea, eb))
+    big = A.clone()
+    big[5] *= 2.0 ** 90
+    big[m - 2] *= 2.0 ** 110
+    check(big, B, "large rows")
+
+
 def test_staged_product_of_very_long_rows(hip):
     """Leading dimensions past the 32-bit load offsets (rows of 2^21 floats)."""
     import torch
