@@ -818,8 +818,9 @@ int small_kind(int64_t batch, int64_t m, int64_t n, int64_t k) {
 // dy the staged column sums cost the product more than the separate pass
 // (cfg5: 73.9 -> 74.5 ms per step). Up to 64 rows (or 16384+ columns) the
 // serial sum of the small-layer launch keeps the reference's order. Only
-// products that take staged tiles without the column sum qualify, so dw keeps
-// the bits of the plain product.
+// products of a class that is the same with and without the column sum
+// qualify, so dw keeps the bits of the plain product: not K or U, which with
+// one would be T, K split through the workspace that they do without.
 std::atomic<bool> g_bias_from_dw{true};
 
 bool bias_from_dw(int64_t rows, int64_t in, int64_t out) {
@@ -830,7 +831,8 @@ bool bias_from_dw(int64_t rows, int64_t in, int64_t out) {
     g.m = in;
     g.n = out;
     g.k = rows;
-    return plan_tile(g, 1, true, false) != Tile::K;
+    const Tile tile = plan_tile(g, 1, true, false);
+    return tile != Tile::K && tile != Tile::U;
 }
 
 // ------------------------------------------------------------ timing probe

@@ -713,7 +713,9 @@ def test_colsum_refusals_and_k_zero(hip):
 # ------------------------------------------------------- Linear backward in one call
 
 @pytest.mark.parametrize("rows,inp,out", [(64, 784, 10), (64, 8, 10), (33, 100, 7),
-                                          (2048, 96, 384), (300, 1024, 257), (100, 3, 20000)])
+                                          (2048, 96, 384), (300, 1024, 257), (100, 3, 20000),
+                                          # dw's plain product on staged tiles with K unsplit
+                                          (1000, 700, 900), (900, 900, 700), (1000, 777, 777)])
 @pytest.mark.parametrize("want", [("dx", "dw", "db"), ("dw", "db"), ("dx",)])
 def test_linear_backward_matches_separate_calls(hip, rows, inp, out, want):
     """ehip_linear_backward_f32 (one launch for small layers) equals the separate
