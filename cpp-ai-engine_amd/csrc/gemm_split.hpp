@@ -383,6 +383,11 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
         if (k_begin < m0) k_begin = k_end < m0 ? k_end : m0;
     }
 
+    // The signs of the steps count from the chunk's first k, so that a product that skips k
+    // keeps those of the product that does not (BM and the chunks are multiples of a step).
+    const int step0 = __builtin_amdgcn_readfirstlane(
+        int((k_begin - int64_t(split) * g.k_chunk) / kSplitBK));
+
     const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
     const int wm0 = (wave / (BN / WN)) * WM, wn0 = (wave % (BN / WN)) * WN;
 
@@ -432,7 +437,7 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
     const auto convert = [&](int s) {
         char* st = lds + (STAGES == 2 ? (s & 1) * kStage : 0);
         ta.store(st, split_scale(0));
-        tb.store(st + 3 * A::kPlane, split_scale(s));
+        tb.store(st + 3 * A::kPlane, split_scale(step0 + s));
         if constexpr (COLSUM) {
 #pragma unroll
             for (int u = 0; u < B::kUnits; ++u) {
@@ -445,7 +450,7 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
         const char* st = lds + (STAGES == 2 ? (s & 1) * kStage : 0);
         split_products<FM, FN, A::kPlane, B::kPlane>(
             acc, st + (wm0 / 16) * 1024 + fbase,
-            st + 3 * A::kPlane + (wn0 / 16) * 1024 + fbase, s);
+            st + 3 * A::kPlane + (wn0 / 16) * 1024 + fbase, step0 + s);
     };
 
     // Two stages: while a step's products run, the next step is converted into the other stage

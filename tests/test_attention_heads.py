@@ -772,14 +772,17 @@ def test_linear_backward_matches_separate_calls(hip, rows, inp, out, want):
 
 # ------------------------------------------------------- causal skipping
 
-@pytest.mark.parametrize("S,hd,bt", [(512, 64, 32), (256, 32, 64), (300, 64, 48)])
+@pytest.mark.parametrize("S,hd,bt", [(512, 64, 32), (256, 32, 64), (300, 64, 48),
+                                     # K split into chunks of an odd number of 32-k steps
+                                     (2048, 64, 4), (296, 64, 1), (516, 64, 1)])
 def test_causal_skipping_modes(hip, S, hd, bt):
     """ehip_gemm_ex_t::causal on batched head products: with P zero above the diagonal,
     P V (mode 2) and P^T G (mode 3) give the bits of the full products; Q K^T with the mask
     (mode 1, scale and mask in the epilogue) and G V^T (mode 1, no epilogue) give the full
     products' bits on and below the diagonal, and above it either those or the epilogue of
     zero (the mask value, or 0). 300 is not a multiple of the tiles (edge checks); the
-    batch counts are large enough for every product to take the staged tiles."""
+    first three batch counts are large enough for every product to take the staged tiles with
+    K unsplit, the others small enough for mode 3's to split K inside the skipped range."""
     print_case("causal modes", S, hd, bt)
     r = np.random.default_rng(S + hd)
     q, k, v, g = (randn(r, bt, S, hd) for _ in range(4))
