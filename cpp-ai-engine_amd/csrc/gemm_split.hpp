@@ -14,9 +14,10 @@
 // Error, against 64-bit products (2-norms; normal operands): K = 64 4.6e-8, K = 1024 1.13e-7,
 // K = 4096 2.1e-7, where the chain of v_mfma_f32_32x32x2f32 that it replaces has 1.4e-7, 5.7e-7
 // and 1.15e-6 (half-normal operands, half of them zero: 4.4e-8, 1.12e-7, 2.1e-7 against 1.0e-7,
-// 4.0e-7 and 8.1e-7); the mean over a column is off by 1.7e-9 of the results' rms, against 3e-9
-// to 6e-9. A step's 32 k are summed apart from the accumulator and by turns negated
-// (split_products, split_flip); all nine part products would give the same figures.
+// 4.0e-7 and 8.1e-7); the mean over a column of 2048 is off by 1.0e-9 of the results' rms at K = 64
+// and 2.0e-9 at K = 1024, against 3.3e-9 and 9.2e-9. A step's 32 k are summed apart from the
+// accumulator (split_products) and their losses made to cancel (split_flip); all nine part products
+// would give the same figures.
 //
 // What bounds it: the matrix pipe at the clock the chip sustains. The bare instruction reaches
 // 1,950 TFLOP/s of its 2,500, i.e. 325 fp32 TFLOP/s with six products; 8192 x 1024 x 4096 runs
@@ -68,6 +69,23 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t& h, uint32
 }
 
 constexpr int kSplitBK = 32;
+
+// The sign bit for odd n. The matrix instruction drops the low bits of its sums towards minus
+// infinity, which leaves every result the same fraction of an ulp low. So odd rows of A and odd
+// columns of B are staged negated, and in odd K steps all of B, and the sums added with the
+// product of the three signs: over neighbouring rows, columns and steps the losses cancel (mean
+// of 2048 x 2048 results' errors over the results' rms, at K = 32, with the sign of odd steps
+// alone -6.1e-9, so less than its own spread, 2e-11; of operands of one sign -2.3e-9, so
+// -1.2e-10).
+__device__ __forceinline__ uint32_t split_flip(int n) { return uint32_t(n) << 31; }
+
+// What an operand is multiplied by as it is split: 2^24, which keeps the parts of the smallest
+// values inside bf16's range (without it a part is lost from |x| < 2^-110 on: a row of 2^-122
+// among rows of 1 kept 13 bits) for about 1 % of the time (8192 x 1024 x 4096 with both its
+// backward products 1039 -> 1050 us). A takes split_scale(0), B split_scale(step).
+__device__ __forceinline__ float split_scale(int s) {
+    return __builtin_bit_cast(float, 0x4b800000u ^ split_flip(s));
+}
 
 // One operand's tile of ROWS rows (of op(A), or columns of op(B)) by 32 k. KC: element (r, k)
 // is at p[r * ld + k], else at p[k * ld + r]. A thread stages kUnits units of one row by 8
@@ -145,8 +163,11 @@ struct SplitTile {
             }
         }
     }
-    // Splits the registers, times `scale` (split_scale), into the three planes.
+    // Splits the registers, times `scale` (split_scale) and negated in odd rows, into the three
+    // planes. A thread's units are rows of one parity.
     __device__ __forceinline__ void store(char* lds, float scale) const {
+        static_assert(THREADS % 8 == 0 && ROWS % 2 == 0, "rows of one parity");
+        scale = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, scale) ^ split_flip(row(0)));
 #pragma unroll
         for (int u = 0; u < kUnits; ++u) {
             uintx4 h, m, l;
@@ -166,23 +187,6 @@ struct SplitTile {
     }
 };
 
-// The sign bit in odd K steps. The matrix instruction drops the low bits of its sums towards
-// minus infinity, which leaves every result the same fraction of an ulp low (3.4e-8 of their
-// rms at K = 1024): odd steps stage B negated and are subtracted, and the two cancel.
-__device__ __forceinline__ uint32_t split_flip(int s) { return uint32_t(s) << 31; }
-
-// What an operand is multiplied by as it is split: 2^24, which keeps the parts of the smallest
-// values inside bf16's range (without it a part is lost from |x| < 2^-110 on: a row of 2^-122
-// among rows of 1 kept 13 bits) for about 1 % of the time (8192 x 1024 x 4096 with both its
-// backward products 1039 -> 1050 us). A takes split_scale(0), B split_scale(s).
-__device__ __forceinline__ float split_scale(int s) {
-    return __builtin_bit_cast(float, 0x4b800000u ^ split_flip(s));
-}
-// What a step's sum is multiplied by as it is added to the accumulator: 2^-48.
-__device__ __forceinline__ float split_unscale(int s) {
-    return __builtin_bit_cast(float, 0x27800000u ^ split_flip(s));
-}
-
 // One staged K step (s) of a wave: acc += its 16 FM x 16 FN tile over 32 k; sa and sb are the
 // lane's place in the first block of the operands' h planes. One block row of A at a time (all
 // of them at once spill in the shapes that run three and four waves per SIMD). Smallest part
@@ -193,7 +197,9 @@ __device__ __forceinline__ float split_unscale(int s) {
 template <int FM, int FN, int PLANE_A, int PLANE_B>
 __device__ __forceinline__ void split_products(floatx4 (&acc)[FM][FN], const char* sa,
                                                const char* sb, int s) {
-    const float unscale = split_unscale(s);
+    // 2^-48, with the sign of the step, of the lane's row of A and of its even columns of B.
+    const float unscale =
+        __builtin_bit_cast(float, 0x27800000u ^ split_flip(s ^ int(threadIdx.x)));
     constexpr int kPart[6][2] = {{1, 1}, {2, 0}, {0, 2}, {0, 1}, {1, 0}, {0, 0}};
     constexpr int SUMS = 2;
     bf16x8 fb[3][FN];
@@ -223,7 +229,8 @@ __device__ __forceinline__ void split_products(floatx4 (&acc)[FM][FN], const cha
             for (int j = 0; j < SUMS; ++j)
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    acc[i][j0 + j][r] = __builtin_fmaf(t[j][r], unscale, acc[i][j0 + j][r]);
+                    acc[i][j0 + j][r] =
+                        __builtin_fmaf(t[j][r], r % 2 ? -unscale : unscale, acc[i][j0 + j][r]);
         }
     }
 }
