@@ -959,7 +959,7 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void co
         split_products<FM, FN, A::kPlane, B::kPlane>(acc, sa, sb, s);
         __syncthreads();
     }
-    if (split_failed<kWaves>(acc, lds)) {
+    if (g.k < kSplitMinK || split_failed<kWaves>(acc, lds)) {
         clear();
 #pragma unroll 1
         for (int64_t k = k_begin; k < k_end; k += 4) {

@@ -69,6 +69,11 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t& h, uint32
 }
 
 constexpr int kSplitBK = 32;
+// Products of fewer k are formed by the fp32 instructions: one or two roundings there, where the
+// dropped parts and the sums' truncation cost more (error against 64 bits at K = 1 2.5e-8 :
+// 3.4e-8, K = 2 3.1e-8 : 3.4e-8, K = 3 of half-normal operands 3.0e-8 : 3.2e-8, from K = 4 on
+// smaller in parts, 4.0e-8 : 3.2e-8).
+constexpr int kSplitMinK = 4;
 
 // The sign bit for odd n. The matrix instruction drops the low bits of its sums towards minus
 // infinity, which leaves every result the same fraction of an ulp low. So odd rows of A and odd
@@ -502,7 +507,7 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
         }
     }
 
-    if (split_failed<kWaves>(acc, lds)) {
+    if (g.k < kSplitMinK || split_failed<kWaves>(acc, lds)) {
         clear();
 #pragma unroll 1
         for (int64_t k = k_begin; k < k_end; k += 4) {

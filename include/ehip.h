@@ -210,7 +210,7 @@ int ehip_memcpy_d2d(void* dst, const void* src, size_t bytes, void* stream);
  * when trans_a != 0; likewise op(B) is k x n. stride_* is the element distance
  * between batch matrices; 0 shares one matrix across the batch (the reference's
  * unbatched operand). beta == 0 overwrites C without reading it.
- * Large products run on the bf16 matrix instructions with each fp32 operand in
+ * Large products of 4 or more k run on the bf16 matrix instructions, each operand in
  * three bf16 parts (24 bits, exact for normal and subnormal values) and fp32
  * accumulation, small ones on the fp32 instructions; either way the result is
  * that of an fp32 product, its error against 64 bits no larger than the fp32

@@ -302,3 +302,12 @@ def test_conv_igemm_wide_ranges(hip, shape, co, k, stride, pad, ew, ex, eg):
             # a subnormal's last bit for each addition beside the bound
             worst = float(np.max(np.abs(host(t).astype(np.float64) - e) / (bound + n * 2.0 ** -149)))
             assert worst <= 1.0, (what, worst)
+
+
+def test_conv_igemm_weight_gradient_of_one_term(hip):
+    """One image, one output pixel: every weight's gradient is one rounded product."""
+    print_case("conv-igemm-one-term")
+    r = np.random.default_rng(3)
+    x, w, g = randn(r, 1, 40, 3, 3), randn(r, 65, 40, 3, 3), randn(r, 1, 65, 1, 1)
+    _, dw, _ = hip.conv2d_igemm_backward(dev(x), dev(w), dev(g), 1, 0)
+    exact(host(dw), g.reshape(65, 1, 1, 1) * x, "dweight")

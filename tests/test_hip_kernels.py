@@ -1310,6 +1310,33 @@ def test_staged_products_are_unbiased(hip, ta, tb, k, positive):
     assert column <= 1.25 * rms / 2048 ** 0.5, (column * 2048 ** 0.5 / rms)
 
 
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("k", [1, 2, 3])
+@pytest.mark.parametrize("positive", [False, True])
+def test_staged_products_of_few_terms(hip, ta, tb, k, positive):
+    """K = 1 is the rounded product of the operands, K = 2 and 3 no further from 64 bits than a
+    chain of fused multiply-adds (emulated in 64 bits)."""
+    import torch
+    print_case("staged few terms", ta, tb, k, positive)
+    g = torch.Generator(device="cuda").manual_seed(k)
+    a = torch.randn(2048, k, device="cuda", generator=g)
+    b = torch.randn(k, 2050, device="cuda", generator=g)
+    if positive:
+        a, b = torch.relu(a), b.abs()
+    got = hip.gemm(a.t().contiguous() if ta else a, b.t().contiguous() if tb else b, trans_a=ta,
+                   trans_b=tb)
+    if k == 1:
+        exact(host(got), host(a * b), "one term")
+        return
+    a, b = a.double(), b.double()
+    chain = torch.zeros(2048, 2050, device="cuda")
+    for i in range(k):
+        chain = (chain.double() + a[:, i:i + 1] * b[i:i + 1]).float()
+    want = a @ b
+    rms = lambda c: float(((c.double() - want) ** 2).mean().sqrt())  # noqa: E731
+    assert rms(got) <= 1.01 * rms(chain), (rms(got), rms(chain))
+
+
 def test_staged_product_of_very_long_rows(hip):
     """Leading dimensions past the 32-bit load offsets (rows of 2^21 floats)."""
     import torch
