@@ -153,18 +153,40 @@ struct SplitTile {
     }
     // The same for a tile of which only the first `left` k are in the matrix (zeros after
     // them), with 64-bit offsets: the last step of a K that is no multiple of 32, and every
-    // step where a leading dimension is too large for offsets().
+    // step where a leading dimension is too large for offsets(). Units wholly inside load as
+    // above (KC): a K of 16 or 24 is one such step (18 x 242 x 242 x 16, A B^T: 9.0 -> 6.9 us).
     __device__ __forceinline__ void load_tail(global_bytes base, int64_t ld, int64_t rows_left,
                                               int left) {
 #pragma unroll
         for (int u = 0; u < kUnits; ++u) {
             const int64_t r = row(u) < rows_left ? row(u) : rows_left - 1;
+            const int in = left - 8 * group(u);
+            if constexpr (KC) {
+                const global_bytes p = base + 4 * (r * ld + 8 * group(u));
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int k = 8 * group(u) + j;
-                const int64_t kk = k < left ? k : 0;
-                const float x = global_load<float>(base + 4 * (KC ? r * ld + kk : kk * ld + r));
-                v[u][j] = k < left ? x : 0.0f;
+                for (int j = 0; j < 8; ++j) v[u][j] = 0.0f;
+                if (in >= 8) {
+                    const floatx4u x = global_load<floatx4u>(p);
+                    const floatx4u y = global_load<floatx4u>(p + 16);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        v[u][j] = x[j];
+                        v[u][4 + j] = y[j];
+                    }
+                } else if (in > 0) {
+#pragma unroll
+                    for (int j = 0; j < 7; ++j) {
+                        const float x = global_load<float>(p + 4 * (j < in ? j : 0));
+                        v[u][j] = j < in ? x : 0.0f;
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const int64_t k = j < in ? 8 * group(u) + j : 0;
+                    const float x = global_load<float>(base + 4 * (k * ld + r));
+                    v[u][j] = j < in ? x : 0.0f;
+                }
             }
         }
     }

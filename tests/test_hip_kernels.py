@@ -1168,6 +1168,9 @@ def test_nt_pipeline_matches_staged_tiles(hip, m, n, k, epi):
 @pytest.mark.parametrize("m,n,k", [(2048, 2049, 1), (1030, 2050, 33), (257, 1281, 300),
                                    (129, 4095, 517), (1999, 777, 1531), (4097, 130, 2049),
                                    (100, 257, 3000),
+                                   # one step, partly in: whole and broken units of eight k
+                                   (2048, 2049, 8), (2047, 2050, 15), (2048, 2051, 16),
+                                   (2049, 2048, 24), (2050, 2047, 31),
                                    # either side of 256 and of 448 tiles of 32 x 32, and of 64 k:
                                    # K sliced over the waves, or staged with K unsplit
                                    (8192, 21, 65), (8193, 21, 64), (8193, 31, 801),
