@@ -500,10 +500,12 @@ int operand_alignment(const GemmArgs& g) {
 //     97 8.2 : 7.2) and, of aligned rows, A^T B^T (800 x 516 x 152 8.0 : 8.7) and the others
 //     at short K (A B 552 x 472 x 152 7.2 : 8.6, x 1012 25.9 : 26.1);
 //   - beyond, none (900 x 700 x 2031: A B 98 : 49, A B^T 142 : 48).
-// Causal products keep the bits of the full product either way.
+// The two sum in different orders, so the rule goes by the shape alone ("aligned rows": those of
+// operands stored without gaps), not by addresses or leading dimensions: a product's bits do not
+// depend on where its operands lie. Causal products keep the bits of the full product either way.
 bool kslice_wins(const GemmArgs& g, int64_t batch, bool ta, bool tb) {
-    const bool rows = operands_aligned(g);
-    if (rows && g.m % 32 == 0 && g.n % 32 == 0 && g.k % 32 == 0)
+    const bool rows = (ta ? g.m : g.k) % 4 == 0 && (tb ? g.k : g.n) % 4 == 0;
+    if (g.m % 32 == 0 && g.n % 32 == 0 && g.k % 32 == 0)
         return double(g.m) * double(g.n) * double(g.k) * double(batch) < 1.2e9;
     const int64_t tiles = ceil_div(g.m, 32) * ceil_div(g.n, 32) * batch;
     if (tiles > 448) return false;

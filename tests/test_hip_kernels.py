@@ -1340,6 +1340,31 @@ def test_staged_products_of_few_terms(hip, ta, tb, k, positive):
     assert rms(got) <= 1.01 * rms(chain), (rms(got), rms(chain))
 
 
+@pytest.mark.parametrize("ta,tb,m,n,k", [(False, False, 552, 472, 152), (False, True, 552, 472, 152),
+                                         (True, True, 800, 516, 152), (False, True, 4096, 64, 64),
+                                         (True, False, 1024, 512, 512), (False, False, 1999, 778, 331),
+                                         (False, False, 2048, 2048, 96)])
+def test_products_bits_by_shape(hip, ta, tb, m, n, k):
+    """The bits of a product depend on its shape: not on the alignment of its operands nor on
+    their leading dimensions."""
+    import torch
+    print_case("bits by shape", ta, tb, m, n, k)
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a = torch.randn((k, m) if ta else (m, k), device="cuda", generator=g)
+    b = torch.randn((n, k) if tb else (k, n), device="cuda", generator=g)
+    want = host(hip.gemm(a, b, trans_a=ta, trans_b=tb))
+    for offset, gap in ((1, 0), (0, 1), (2, 5)):
+        def moved(t):
+            flat = torch.zeros(offset + t.shape[0] * (t.shape[1] + gap), device="cuda")
+            v = flat[offset:].view(t.shape[0], t.shape[1] + gap)
+            v[:, :t.shape[1]] = t
+            return v
+        x, y, c = moved(a), moved(b), hip.f32((m, n))
+        hip.ok(hip.lib.ehip_gemm_f32(int(ta), int(tb), 1, m, n, k, hip.p(x), x.shape[1], 0, hip.p(y),
+                                     y.shape[1], 0, 0.0, hip.p(c), n, 0, hip.stream()), "gemm")
+        exact(host(c), want, f"offset {offset}, gap {gap}")
+
+
 def test_staged_product_of_very_long_rows(hip):
     """Leading dimensions past the 32-bit load offsets (rows of 2^21 floats)."""
     import torch
