@@ -499,7 +499,16 @@ int operand_alignment(const GemmArgs& g) {
 //   - to 448 tiles, A^T B (rows of both operands contiguous: 11000 x 31 x 1021 25 : 28.5, but x
 //     97 8.2 : 7.2) and, of aligned rows, A^T B^T (800 x 516 x 152 8.0 : 8.7) and the others
 //     at short K (A B 552 x 472 x 152 7.2 : 8.6, x 1012 25.9 : 26.1);
-//   - beyond, none (900 x 700 x 2031: A B 98 : 49, A B^T 142 : 48).
+//   - to 512, two per CU, A^T B of long K (3825 x 104 x 1651 38.3 : 43.5, 668 x 757 x 484 15.3 :
+//     16.5; 179 x 2523 x 436 15.4 : 14.8, and beyond 512 a third round, 172 x 2852 x 1090 0.67 of
+//     the sliced time);
+//   - beyond, none (900 x 700 x 2031: A B 98 : 49, A B^T 142 : 48), but for batches of matrices of
+//     up to 32 rows over one staged step: half of every 64 x 64 tile is empty there, or five
+//     eighths of columns that end in the first half of a tile, and from 768 tiles (three per CU,
+//     one round), or 512, the sliced ones do less (400 x (31 x 72 x 31) 8.2 : 9.8, 390 x
+//     (14 x 120 x 14) 7.9 : 9.3, 305 x (19 x 96 x 19) 6.8 : 7.5; 329 x (14 x 127 x 14) 7.8 : 7.1);
+//     and for batches of more than 512 results of A B^T of up to 24 x 24 (672 x (14 x 14 x 72)
+//     7.8 : 9.2, 611 x (23 x 23 x 88) 8.5 : 9.5; 560 x (26 x 26 x 96) 8.9 : 8.4).
 // The two sum in different orders, so the rule goes by the shape alone ("aligned rows": those of
 // operands stored without gaps), not by addresses or leading dimensions: a product's bits do not
 // depend on where its operands lie. Causal products keep the bits of the full product either way.
@@ -508,7 +517,12 @@ bool kslice_wins(const GemmArgs& g, int64_t batch, bool ta, bool tb) {
     if (g.m % 32 == 0 && g.n % 32 == 0 && g.k % 32 == 0)
         return double(g.m) * double(g.n) * double(g.k) * double(batch) < 1.2e9;
     const int64_t tiles = ceil_div(g.m, 32) * ceil_div(g.n, 32) * batch;
-    if (tiles > 448) return false;
+    if (tiles > 448) {
+        const int64_t staged = ceil_div(g.m, 64) * ceil_div(g.n, 64) * batch;
+        if (g.m <= 32 && g.k <= 32) return staged > (8 * tiles <= 12 * staged ? 512 : 768);
+        if (!ta && tb && g.m <= 24 && g.n <= 24) return tiles > 512;
+        return ta && !tb && batch == 1 && tiles <= 512 && g.k > 480;
+    }
     if (!ta && rows) return tiles <= 256 || g.k <= (tb ? 256 : 512);
     if (!ta && tb) return tiles < 100 ? g.k > 64 : tiles <= 256 && g.k > 96 && g.k <= 256;
     if (tiles <= 256 || (ta && tb && rows)) return g.k > 64;

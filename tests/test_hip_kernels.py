@@ -1340,6 +1340,30 @@ def test_staged_products_of_few_terms(hip, ta, tb, k, positive):
     assert rms(got) <= 1.01 * rms(chain), (rms(got), rms(chain))
 
 
+# Either side of the lines at which batches of small matrices, and long A^T B products of up to 512
+# tiles of 32 x 32, go from staged tiles to K-sliced ones.
+@pytest.mark.parametrize("ta,tb,batch,m,n,k", [(False, False, 256, 20, 96, 20), (False, False, 257, 20, 96, 20),
+                                               (True, False, 384, 32, 120, 32), (True, False, 385, 32, 120, 32),
+                                               (False, False, 385, 32, 120, 33), (False, False, 385, 33, 120, 32),
+                                               (False, True, 512, 24, 23, 72), (False, True, 513, 24, 23, 72),
+                                               (False, True, 513, 25, 23, 72),
+                                               (True, False, 1, 3825, 104, 480), (True, False, 1, 3825, 104, 481),
+                                               (True, False, 1, 4096, 125, 481), (True, False, 1, 4097, 124, 481)])
+def test_small_matrices_sliced_or_staged(hip, ta, tb, batch, m, n, k):
+    import torch
+    from _hip import gemm_stat_bound
+    print_case("sliced or staged", ta, tb, batch, m, n, k)
+    g = torch.Generator(device="cuda").manual_seed(batch + m + k)
+    a = torch.randn(batch, k if ta else m, m if ta else k, device="cuda", generator=g)
+    b = torch.randn(batch, n if tb else k, k if tb else n, device="cuda", generator=g)
+    got = hip.gemm(a, b, trans_a=ta, trans_b=tb).double().view(batch, m, n)
+    a, b = a.double(), b.double()
+    a, b = (a.transpose(1, 2) if ta else a).contiguous(), (b.transpose(1, 2) if tb else b).contiguous()
+    want = torch.bmm(a, b)
+    bound = gemm_stat_bound(a.norm(dim=2), b.norm(dim=1), k) + 2.0 ** -22 * want.abs()
+    assert float(((got - want).abs() / bound).max()) <= 1.0
+
+
 @pytest.mark.parametrize("ta,tb,m,n,k", [(False, False, 552, 472, 152), (False, True, 552, 472, 152),
                                          (True, True, 800, 516, 152), (False, True, 4096, 64, 64),
                                          (True, False, 1024, 512, 512), (False, False, 1999, 778, 331),
