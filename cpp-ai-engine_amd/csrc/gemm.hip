@@ -512,7 +512,10 @@ int operand_alignment(const GemmArgs& g) {
 // The two sum in different orders, so the rule goes by the shape alone ("aligned rows": those of
 // operands stored without gaps), not by addresses or leading dimensions: a product's bits do not
 // depend on where its operands lie. Causal products keep the bits of the full product either way.
+// From 2^24 tiles of 64 x 64 (2^30 rows), whose 2^32 threads are more than a launch takes, the
+// sliced ones' single wave per tile still fits.
 bool kslice_wins(const GemmArgs& g, int64_t batch, bool ta, bool tb) {
+    if (ceil_div(g.m, 64) * ceil_div(g.n, 64) >= int64_t(1) << 24) return true;
     const bool rows = (ta ? g.m : g.k) % 4 == 0 && (tb ? g.k : g.n) % 4 == 0;
     if (g.m % 32 == 0 && g.n % 32 == 0 && g.k % 32 == 0)
         return double(g.m) * double(g.n) * double(g.k) * double(batch) < 1.2e9;

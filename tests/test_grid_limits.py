@@ -41,6 +41,23 @@ def test_gemm_batch_beyond_grid(hip, batch, m, n, k):
     exact(got, np.matmul(a, b), "batched product")
 
 
+@pytest.mark.parametrize("m", [(1 << 30) - 64, 1 << 30, (1 << 30) + 4097])
+def test_gemm_rows_to_the_grid_limit(hip, m):
+    """A single column of 2^30 rows, whose 64 x 64 tiles would be 2^32 threads, and its
+    neighbours; integer operands, so exact."""
+    import torch
+    print_case("gemm rows", m)
+    g = torch.Generator(device="cuda").manual_seed(m)
+    a = torch.randint(-4, 5, (m, 2), device="cuda", generator=g, dtype=torch.int8)
+    A, b = a.float(), torch.tensor([[3.0], [-2.0]], device="cuda")
+    c = hip.gemm(A, b)
+    wrong = 0
+    for i in range(0, m, 1 << 27):
+        x = A[i:i + (1 << 27)]
+        wrong += int((c[i:i + (1 << 27), 0] != x[:, 0] * 3.0 - x[:, 1] * 2.0).sum())
+    assert wrong == 0, wrong
+
+
 def test_gemm_ex_two_level_batch_beyond_grid(hip):
     """The extended product with two-level strides (2 heads per sample) and a per-head addend
     and scale in the epilogue over 65538 products: product z reads sample z / 2, head z % 2,
