@@ -1203,13 +1203,20 @@ TapGeo finish_taps(TapGeo tg) {
     return tg;
 }
 
-// Whether dW runs on the split tiles: 32 images of x within 32-bit byte offsets.
-bool takes_runs(const ConvGeo& cg) { return cg.chw < (int64_t(1) << 25) - 1; }
+// The loaders' pixel indices are 32-bit and run past the last pixel to the end of a tile or
+// step, and a step further.
+constexpr int64_t kPixels = INT_MAX - 255;
 
-// Whether a product over `channels` channels may run tap by tap: little padding of the
-// channels, and 32-bit offsets in an image.
-bool takes_taps(int64_t channels, int64_t image) {
-    return channels >= kTapChannels && 4 * image <= 0xffffffffLL;
+// Whether dW over `pixels` output pixels runs on the split tiles: 32 images of x within 32-bit
+// byte offsets.
+bool takes_runs(const ConvGeo& cg, int64_t pixels) {
+    return cg.chw < (int64_t(1) << 25) - 1 && pixels <= kPixels;
+}
+
+// Whether a product of `pixels` results an image over `channels` channels may run tap by tap:
+// little padding of the channels, and 32-bit offsets in a gathered image's channel.
+bool takes_taps(int64_t channels, int64_t in_hw, int64_t pixels) {
+    return channels >= kTapChannels && 4 * in_hw <= 0xffffffffLL && pixels <= kPixels;
 }
 
 // The stride phases of dx (stride 2..4, N s^2 <= 65535 products); false
@@ -1313,7 +1320,7 @@ int ehip_conv2d_igemm_f32(const float* x, const float* weight, const float* bias
     g.add_row = 1;
     g.add_period = 1;
     const hipStream_t s = as_stream(stream);
-    const PackBlock packed(stream, takes_taps(cg.c, cg.hw), int64_t(cg.co) * cg.k);
+    const PackBlock packed(stream, takes_taps(cg.c, cg.hw, cg.p), int64_t(cg.co) * cg.k);
     if (packed.p != nullptr) {
         TapGeo tg{};
         tg.channels = cg.c;
@@ -1366,7 +1373,7 @@ int ehip_conv2d_igemm_backward_f32(const float* x, const float* weight, const fl
         g.inner = 1;
         g.alpha = 1.0f;
         g.add_period = 1;
-        const int rc = takes_runs(cg)
+        const int rc = takes_runs(cg, g.k)
                            ? launch_split<ConvGeo, DoutRows, TapRows>(g, 1, g.k, cg, s)
                            : run_product<DoutByChannel, ColsByTap, false>(g, 1, cg, vec_dout, false, s);
         if (rc) return rc;
@@ -1415,7 +1422,7 @@ int ehip_conv2d_igemm_backward_f32(const float* x, const float* weight, const fl
             if (int rc2 = ehip_gemm_ex_f32(&d, stream)) return rc2;
             return ehip_col2im_f32(dcols, dx, win, stream);
         }
-        const PackBlock packed(stream, cg.stride == 1 && takes_taps(cg.co, cg.p),
+        const PackBlock packed(stream, cg.stride == 1 && takes_taps(cg.co, cg.p, cg.hw),
                                int64_t(cg.co) * cg.k);
         if (packed.p != nullptr) {
             // The input gradient of a stride-1 layer is a convolution of dOut with the taps

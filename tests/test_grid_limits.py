@@ -98,3 +98,25 @@ def test_sum_axis_outer_beyond_grid(hip, orc, outer, axis_len, inner):
     x = np.random.default_rng(outer).standard_normal((outer, axis_len, inner), dtype=np.float32)
     got = host(hip.sum_axis(dev(x), outer, axis_len, inner)).reshape(outer, inner)
     exact(got, orc.sum_axis(x, 1).reshape(outer, inner), "sum_axis")
+
+
+def test_conv_weight_gradient_of_two_to_the_31_pixels(hip):
+    """49981 images of 198 x 217 pixels: 2^31 - 2 in all, the 32-bit reduction index's last few.
+    Integer operands and random signs, so every partial sum is exact."""
+    import torch
+    n, h, w = 49981, 198, 217
+    print_case("conv dweight", n, h, w)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randint(0, 2, (n, 1, h, w), device="cuda", generator=g, dtype=torch.int8)
+    dy = torch.randint(-1, 2, (n, 1, h, w), device="cuda", generator=g, dtype=torch.int8)
+    weight = torch.ones(1, 1, 1, 1, device="cuda")
+    from ehip import window
+    import ctypes
+    X, G, dw, db = x.float(), dy.float(), hip.f32((1, 1, 1, 1)), hip.f32((1,))
+    win = window(n, 1, h, w, 1, 1, 1, 0)
+    hip.ok(hip.lib.ehip_conv2d_igemm_backward_f32(hip.p(X), hip.p(weight), hip.p(G), None, hip.p(dw),
+                                                  hip.p(db), ctypes.byref(win), 1, hip.stream()),
+           "conv2d_igemm_backward")
+    want_w = sum(int((x[i:i + 4096].int() * dy[i:i + 4096]).sum()) for i in range(0, n, 4096))
+    want_b = sum(int(dy[i:i + 4096].int().sum()) for i in range(0, n, 4096))
+    assert (float(dw[0, 0, 0, 0]), float(db[0])) == (want_w, want_b)
