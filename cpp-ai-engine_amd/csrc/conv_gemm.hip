@@ -647,6 +647,8 @@ struct TapGeo {
     int64_t image;         // channels h w
     const float* in;
     const float* packed;
+    const float* weight;  // where there is no packed block (WeightTaps)
+    int64_t row_pitch, channel_pitch, tap_pitch;
     FastDiv d_ow;
 };
 
@@ -720,6 +722,46 @@ struct PackedRows : SplitTile<ROWS, true, THREADS> {
         const int t = int(k / g.padded), c = int(k - int64_t(t) * g.padded);
         if (r >= rows_left || c >= g.channels) return 0.0f;
         return g.packed[((r0 + r) * g.kh * g.kw + t) * g.channels + c];
+    }
+};
+
+// The same rows from the weights as they are: element (r, c) of tap t is at
+// weight[r row_pitch + c channel_pitch + t tap_pitch]. The values, and so the results' bits, are
+// those of the packed rows.
+template <int ROWS, int THREADS>
+struct WeightTaps : SplitTile<ROWS, true, THREADS> {
+    using T = SplitTile<ROWS, true, THREADS>;
+    const TapGeo& g;
+    int64_t r0, rows_left;
+    int tap, c0;
+    __device__ WeightTaps(const TapGeo& g_, int64_t, int64_t r0_, int64_t rows, int64_t k0, int64_t)
+        : g(g_), r0(r0_), rows_left(rows - r0_) {
+        tap = int(k0 / g.padded);
+        c0 = int(k0 - int64_t(tap) * g.padded);
+    }
+    __device__ __forceinline__ void next() {
+#pragma unroll
+        for (int u = 0; u < T::kUnits; ++u) {
+            const int64_t r = T::row(u) < rows_left ? T::row(u) : rows_left - 1;
+            const auto row = (global_bytes)(g.weight + (r0 + r) * g.row_pitch + tap * g.tap_pitch);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int c = c0 + 8 * T::group(u) + j;
+                const float x =
+                    global_load<float>(row + 4 * g.channel_pitch * min(c, g.channels - 1));
+                this->v[u][j] = c < g.channels ? x : 0.0f;
+            }
+        }
+        c0 += 32;
+        if (c0 >= g.padded) {
+            c0 = 0;
+            ++tap;
+        }
+    }
+    __device__ float at(int r, int64_t k) const {
+        const int t = int(k / g.padded), c = int(k - int64_t(t) * g.padded);
+        if (r >= rows_left || c >= g.channels) return 0.0f;
+        return g.weight[(r0 + r) * g.row_pitch + c * g.channel_pitch + t * g.tap_pitch];
     }
 };
 
@@ -1160,11 +1202,11 @@ int run_product(const GemmArgs& g, int64_t batch, const ConvGeo& cg, bool vec_a,
     return launch_product<Small, 16, LA, LB, EPI>(g, batch, cg, vec_a, vec_b, s);
 }
 
-// A call's own block for the packed weights (null: the product takes the gather kernels, which
-// need none). The library's scratch would be shared by calls that overlap on several streams or
-// threads. The arena's blocks are ordered with the null stream (or the calling thread's
-// capture), so only calls there take one; kPackFloats (64 MiB) holds 1024 x 1024 x 3 x 3 and
-// keeps what a call asks for beside its operands small.
+// A call's own block for the packed weights (null: the weights are read as they are). The
+// library's scratch would be shared by calls that overlap on several streams or threads. The
+// arena's blocks are ordered with the null stream (or the calling thread's capture), so only calls
+// there take one; kPackFloats (64 MiB) holds 1024 x 1024 x 3 x 3 and keeps what a call asks for
+// beside its operands small. Either way the same bits.
 constexpr int64_t kPackFloats = int64_t(1) << 24;
 struct PackBlock {
     void* p = nullptr;
@@ -1179,20 +1221,37 @@ struct PackBlock {
     float* data() const { return static_cast<float*>(p); }
 };
 
-// The tap-by-tap product (forward; dx with FLIP): repacks the weights, then the split tiles.
-// `g` carries m, n, c and the epilogue.
+// The multiply-adds times taps from which packed weights pay for their launch (5 us). Read as they
+// are, one tap of a row lies `taps` floats apart, so the loads grow with the taps. Forward and dx
+// together, packed : as they are (us): 3 x 3, 5 x 53 -> 41 channels of 47 x 47 (2.2e8 multiply-adds
+// each) 80.8 : 78.4, 13 x 254 -> 29 of 17 x 17 (2.5e8) 78.7 : 80.9, 19 x 182 -> 168 of 15 x 15
+// (1.2e9) 153 : 181; 5 x 5, 53 -> 30 of 43 x 43 (7.4e7) 56.6 : 51.5, 3 x 58 -> 32 of 32 x 32
+// (1.4e8) 56.3 : 60.5, 49 x 96 -> 121 of 12 x 12 (2.1e9) 263 : 490. A 1 x 1 kernel's rows are
+// contiguous as they are (28 x 130 -> 86 of 46 x 46 128 : 126).
+constexpr double kPackWork = 2e9;
+
+// The tap-by-tap product (forward; dx with FLIP) on the split tiles. `g` carries m, n, c and the
+// epilogue.
 template <bool FLIP>
-int run_taps(GemmArgs g, int64_t batch, TapGeo tg, const float* weight, float* packed,
-             hipStream_t s) {
+int run_taps(GemmArgs g, int64_t batch, TapGeo tg, const float* weight, void* stream) {
     const int taps = tg.kh * tg.kw;
-    const int64_t total = g.m * taps * tg.channels;  // at most kPackFloats
-    EHIP_LAUNCH("conv_pack_weights", conv_pack_weights<FLIP>, dim3(unsigned(ceil_div(total, 256))),
-                dim3(256), 0, s, weight, packed, total, tg.channels, taps, fast_div(tg.channels),
-                fast_div(taps));
-    tg.packed = packed;
+    const int64_t total = g.m * taps * tg.channels, k = int64_t(taps) * tg.channels;
+    const hipStream_t s = as_stream(stream);
     g.k = int64_t(taps) * tg.padded;
-    return launch_split<TapGeo, PackedRows, TapPixels>(g, batch, int64_t(taps) * tg.channels, tg,
-                                                       s);
+    const double work = double(g.m) * double(g.n) * double(batch) * double(k);
+    const PackBlock packed(stream, taps > 1 && work * taps >= kPackWork, total);
+    if (packed.p == nullptr) {
+        tg.weight = FLIP ? weight + taps - 1 : weight;
+        tg.row_pitch = FLIP ? taps : k;
+        tg.channel_pitch = FLIP ? g.m * taps : taps;
+        tg.tap_pitch = FLIP ? -1 : 1;
+        return launch_split<TapGeo, WeightTaps, TapPixels>(g, batch, k, tg, s);
+    }
+    EHIP_LAUNCH("conv_pack_weights", conv_pack_weights<FLIP>, dim3(unsigned(ceil_div(total, 256))),
+                dim3(256), 0, s, weight, packed.data(), total, tg.channels, taps,
+                fast_div(tg.channels), fast_div(taps));
+    tg.packed = packed.data();
+    return launch_split<TapGeo, PackedRows, TapPixels>(g, batch, k, tg, s);
 }
 
 TapGeo finish_taps(TapGeo tg) {
@@ -1320,8 +1379,7 @@ int ehip_conv2d_igemm_f32(const float* x, const float* weight, const float* bias
     g.add_row = 1;
     g.add_period = 1;
     const hipStream_t s = as_stream(stream);
-    const PackBlock packed(stream, takes_taps(cg.c, cg.hw, cg.p), int64_t(cg.co) * cg.k);
-    if (packed.p != nullptr) {
+    if (takes_taps(cg.c, cg.hw, cg.p)) {
         TapGeo tg{};
         tg.channels = cg.c;
         tg.h = cg.h;
@@ -1333,7 +1391,7 @@ int ehip_conv2d_igemm_f32(const float* x, const float* weight, const float* bias
         tg.kh = cg.kh;
         tg.kw = cg.kw;
         tg.in = x;
-        return run_taps<false>(g, win->batch, finish_taps(tg), weight, packed.data(), s);
+        return run_taps<false>(g, win->batch, finish_taps(tg), weight, stream);
     }
     const bool vec_w = cg.k % 4 == 0 && aligned16(weight);
     if (bias) return run_product<WeightRows, ColsByPixel, true>(g, win->batch, cg, vec_w, false, s);
@@ -1422,9 +1480,7 @@ int ehip_conv2d_igemm_backward_f32(const float* x, const float* weight, const fl
             if (int rc2 = ehip_gemm_ex_f32(&d, stream)) return rc2;
             return ehip_col2im_f32(dcols, dx, win, stream);
         }
-        const PackBlock packed(stream, cg.stride == 1 && takes_taps(cg.co, cg.p, cg.hw),
-                               int64_t(cg.co) * cg.k);
-        if (packed.p != nullptr) {
+        if (cg.stride == 1 && takes_taps(cg.co, cg.p, cg.hw)) {
             // The input gradient of a stride-1 layer is a convolution of dOut with the taps
             // reversed and the padding kH - 1 - pad.
             TapGeo tg{};
@@ -1439,7 +1495,7 @@ int ehip_conv2d_igemm_backward_f32(const float* x, const float* weight, const fl
             tg.kh = cg.kh;
             tg.kw = cg.kw;
             tg.in = grad_out;
-            rc = run_taps<true>(g, n, finish_taps(tg), weight, packed.data(), s);
+            rc = run_taps<true>(g, n, finish_taps(tg), weight, stream);
         } else if (cg.stride == 1)
             rc = run_product<WeightByInput, DoutByPixelS1, false>(g, n, cg, false, false, s);
         else if (!plan_phases(cg, n, &ps, &phases, &max_count))

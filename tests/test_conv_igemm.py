@@ -215,9 +215,9 @@ def test_conv_igemm_empty_batch_and_errors(hip):
                                                    ((1, 40, 5, 9), 70, 1, 1, 0),
                                                    ((2, 65, 12, 14), 130, 5, 1, 2)])
 def test_conv_igemm_tap_edges(hip, shape, co, k, stride, pad):
-    """On the null stream (tap by tap from 24 channels on) and on a named one (the gather kernels,
-    which need no packed weights): both within the worst-case fp32 bound of the exact product, and
-    an infinite input reaches the same outputs."""
+    """On the null stream (weights packed in a block of the call's own) and on a named one (read as
+    they are): the same bits, within the worst-case fp32 bound of the exact product, and an infinite
+    input reaches the same outputs."""
     import torch
     print_case("conv-igemm-taps", shape, co, k, stride, pad)
     r = np.random.default_rng(sum(shape) + co + k)
@@ -242,9 +242,12 @@ def test_conv_igemm_tap_edges(hip, shape, co, k, stride, pad):
         within(host(DX), ex[1], "dx")
         within(host(DW), ex[2], "dweight")
         within(host(DB), ex[3], "dbias")
-        reached.append(host(YB))
-    exact(np.isfinite(reached[0]).astype(np.float32), np.isfinite(reached[1]).astype(np.float32),
-          "outputs of an infinite input")
+        reached.append([host(t) for t in (Y, DX, DW, DB, YB)])
+    for i, what in enumerate(("forward", "dx", "dweight", "dbias")):
+        exact(reached[1][i], reached[0][i], f"{what} on a named stream")
+    yb = exact_products(np.nan_to_num(bad), w, b, g, stride, pad)[0][0]
+    assert np.array_equal(np.isfinite(reached[0][4]), np.isfinite(reached[1][4]))
+    assert np.array_equal(np.isfinite(reached[0][4]), np.abs(yb) < 1e30), "outputs of an infinite input"
 
 
 @pytest.mark.parametrize("kind", ["conv", "product"])
