@@ -55,6 +55,7 @@ public:
     std::vector<float>& host_mut();
 
     bool resident_on_device() const noexcept;
+    bool resident_on_host() const noexcept;
     // True when no other Storage shares this buffer. The engine mutates a
     // buffer in place only when it is exclusive (gradient buffers may be
     // shared after add_grad adopts a temporary).

@@ -115,6 +115,7 @@ std::vector<float>& Storage::host_mut() {
 }
 
 bool Storage::resident_on_device() const noexcept { return buf_ && buf_->device_valid; }
+bool Storage::resident_on_host() const noexcept { return buf_ && buf_->host_valid; }
 
 uint64_t Storage::version() const noexcept { return buf_ ? buf_->version : 0; }
 

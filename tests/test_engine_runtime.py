@@ -112,6 +112,29 @@ def test_arena_flat_after_warmup_and_trim(eng, hip):
     assert s.bytes_reserved == s.bytes_in_use
 
 
+@pytest.mark.parametrize("vocab,d,heads,ff,layers", [(121, 96, 4, 384, 2), (64, 1024, 8, 4096, 1),
+                                                     (300, 512, 8, 1100, 2)])
+def test_parameter_read_back(eng, hip, vocab, d, heads, ff, layers):
+    """Parameters come back in their order and unchanged (steps of a learning rate that moves only
+    the zeros, by 1e-30, put them on the device), whether gathered or one by one, and take at most
+    a 4 MiB block beside them."""
+    print_case("read-back", vocab, d, heads, ff, layers)
+    from engine_capi import Trainer
+    ids, targets = W.lm_inputs(1, 2, 16, vocab)
+    params = W.lm_init_params(2, vocab, d, ff, layers)
+    tr = Trainer.charlm(eng, ids, targets, vocab, d, heads, ff, layers, params, lr=1e-30)
+    for _ in range(2):
+        tr.step()
+    eng.synchronize()
+    hip.ok(hip.lib.ehip_arena_trim(), "trim")
+    before = hip.arena_stats().bytes_reserved
+    got = tr.params()
+    assert got.shape == params.shape and float(np.abs(got - params).max()) <= 3e-30
+    assert hip.arena_stats().bytes_reserved - before <= 4 << 20
+    exact(tr.params(), got, "a second read")
+    tr.close()
+
+
 # ------------------------------------------------------------------ failure injection
 
 def launches_per_step(eng, hip, tr):
