@@ -552,9 +552,12 @@ Tile plan_tile(const GemmArgs& g, int64_t batch, bool ta, bool tb) {
     if (ta && !tb && batch == 1 && g.causal == 0 && g.k >= 1024 &&
         ceil_div(g.m, 16) * ceil_div(g.n, 16) <= 1024)
         return Tile::P;
-    // A B column sum is computed only by the staged tiles.
-    if (g.colsum == nullptr && ceil_div(g.m, 32) * ceil_div(g.n, 32) * batch >= 64)
-        return kslice_wins(g, batch, ta, tb) ? Tile::K : Tile::U;
+    // A B column sum is computed only by the staged tiles: with one, K's sizes are T's, and U's,
+    // whose unsplit tiles form it as well, stay U's.
+    if (ceil_div(g.m, 32) * ceil_div(g.n, 32) * batch >= 64) {
+        if (!kslice_wins(g, batch, ta, tb)) return Tile::U;
+        if (g.colsum == nullptr) return Tile::K;
+    }
     return Tile::T;
 }
 
@@ -838,8 +841,8 @@ int small_kind(int64_t batch, int64_t m, int64_t n, int64_t k) {
 // (cfg5: 73.9 -> 74.5 ms per step). Up to 64 rows (or 16384+ columns) the
 // serial sum of the small-layer launch keeps the reference's order. Only
 // products of a class that is the same with and without the column sum
-// qualify, so dw keeps the bits of the plain product: not K or U, which with
-// one would be T, K split through the workspace that they do without.
+// qualify, so dw keeps the bits of the plain product: not K, which with one
+// would be T.
 std::atomic<bool> g_bias_from_dw{true};
 
 bool bias_from_dw(int64_t rows, int64_t in, int64_t out) {
@@ -850,8 +853,7 @@ bool bias_from_dw(int64_t rows, int64_t in, int64_t out) {
     g.m = in;
     g.n = out;
     g.k = rows;
-    const Tile tile = plan_tile(g, 1, true, false);
-    return tile != Tile::K && tile != Tile::U;
+    return plan_tile(g, 1, true, false) != Tile::K;
 }
 
 // ------------------------------------------------------------ timing probe

@@ -361,8 +361,8 @@ int ehip_gemm_probe_read(double* ms, int64_t* products, double* flop);
  * bit; when all requested parts are small (thread-per-output products, a
  * serial column sum) they run in one launch. db is ehip_sum_axis_f32's, except
  * for mid-sized layers (more than 64 rows, dy of at most 2^21 elements, fewer
- * than 16384 columns, dw requested too, and a dw product of a kind that forms
- * column sums without changing), where it is the column sums of dy that the dw
+ * than 16384 columns, dw requested too, and a dw product that takes staged
+ * MFMA tiles either way), where it is the column sums of dy that the dw
  * product forms from the tiles it stages (ehip_gemm_ex_f32's colsum_b): the
  * same sums in another order, two launches fewer. dx, dw and db may each be
  * NULL. */
