@@ -971,6 +971,7 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void co
     const int64_t k_begin = int64_t(blockIdx.y) * g.k_chunk;
     const int64_t k_end = min(k_begin + g.k_chunk, g.k);
     const int steps = int((k_end - k_begin + kSplitBK - 1) / kSplitBK);
+    const int pairs = split_pairs(k_end - k_begin);
     A a(cg, z, m0, g.m, k_begin, k_end);
     B b(cg, z, n0, g.n, k_begin, k_end);
     const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
@@ -991,14 +992,15 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void co
         b.next();
     }
     for (int s = 0; s < steps; ++s) {
-        a.store(lds, split_scale(0));
-        b.store(lds + 3 * A::kPlane, split_scale(s));
+        const int unpaired = s >= pairs ? -1 : 0;
+        a.store(lds, split_scale(A::T::row(0) & unpaired));
+        b.store(lds + 3 * A::kPlane, split_scale(s ^ (B::T::row(0) & unpaired)));
         if (s + 1 < steps) {
             a.next();
             b.next();
         }
         __syncthreads();
-        split_products<FM, FN, A::kPlane, B::kPlane>(acc, sa, sb, s);
+        split_products<FM, FN, A::kPlane, B::kPlane>(acc, sa, sb, s, unpaired);
         __syncthreads();
     }
     if (g.k < kSplitMinK || split_failed<kWaves>(acc, lds)) {

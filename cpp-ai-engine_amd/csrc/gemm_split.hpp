@@ -76,20 +76,22 @@ constexpr int kSplitBK = 32;
 constexpr int kSplitMinK = 4;
 
 // The sign bit for odd n. The matrix instruction drops the low bits of its sums towards minus
-// infinity, which leaves every result the same fraction of an ulp low. So odd rows of A and odd
-// columns of B are staged negated, and in odd K steps all of B, and the sums added with the
-// product of the three signs: over neighbouring rows, columns and steps the losses cancel (mean
-// of 2048 x 2048 results' errors over the results' rms, at K = 32, with the sign of odd steps
-// alone -6.1e-9, so less than its own spread, 2e-11; of operands of one sign -2.3e-9, so
-// -1.2e-10).
+// infinity, which leaves every result the same fraction of an ulp low: in odd K steps B is staged
+// negated and the sum subtracted, and the losses of a pair of steps cancel. In the steps that are
+// left of a chunk of K after its whole pairs (from split_pairs on), odd rows of A and odd columns of B
+// are negated too and the sums added with the product of the three signs, so that their losses
+// cancel over neighbouring rows and columns (mean of 2048 x 2048 results' errors over the results'
+// rms, at K = 32, with the steps' signs alone -6.1e-9, so less than its own spread, 2e-11; of
+// operands of one sign -2.3e-9, so -1.2e-10).
 __device__ __forceinline__ uint32_t split_flip(int n) { return uint32_t(n) << 31; }
+__device__ __forceinline__ int split_pairs(int64_t chunk) { return int(chunk / kSplitBK) & ~1; }
 
 // What an operand is multiplied by as it is split: 2^24, which keeps the parts of the smallest
 // values inside bf16's range (without it a part is lost from |x| < 2^-110 on: a row of 2^-122
 // among rows of 1 kept 13 bits) for about 1 % of the time (8192 x 1024 x 4096 with both its
-// backward products 1039 -> 1050 us). A takes split_scale(0), B split_scale(step).
-__device__ __forceinline__ float split_scale(int s) {
-    return __builtin_bit_cast(float, 0x4b800000u ^ split_flip(s));
+// backward products 1039 -> 1050 us). With the sign of n: of A's row, or of the step and B's column.
+__device__ __forceinline__ float split_scale(int n) {
+    return __builtin_bit_cast(float, 0x4b800000u ^ split_flip(n));
 }
 
 // One operand's tile of ROWS rows (of op(A), or columns of op(B)) by 32 k. KC: element (r, k)
@@ -190,11 +192,10 @@ struct SplitTile {
             }
         }
     }
-    // Splits the registers, times `scale` (split_scale) and negated in odd rows, into the three
-    // planes. A thread's units are rows of one parity.
+    // Splits the registers, times `scale` (split_scale), into the three planes. A thread's units
+    // are rows of one parity, that of row(0).
     __device__ __forceinline__ void store(char* lds, float scale) const {
         static_assert(THREADS % 8 == 0 && ROWS % 2 == 0, "rows of one parity");
-        scale = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, scale) ^ split_flip(row(0)));
 #pragma unroll
         for (int u = 0; u < kUnits; ++u) {
             uintx4 h, m, l;
@@ -223,10 +224,12 @@ struct SplitTile {
 // error 4.85e-7 -> 1.18e-7, for 3 to 6 % of the time).
 template <int FM, int FN, int PLANE_A, int PLANE_B>
 __device__ __forceinline__ void split_products(floatx4 (&acc)[FM][FN], const char* sa,
-                                               const char* sb, int s) {
-    // 2^-48, with the sign of the step, of the lane's row of A and of its even columns of B.
-    const float unscale =
-        __builtin_bit_cast(float, 0x27800000u ^ split_flip(s ^ int(threadIdx.x)));
+                                               const char* sb, int s, int unpaired) {
+    // 2^-48, with the sign of the step, of the lane's row of A and of its even or odd columns of B.
+    const float even = __builtin_bit_cast(
+        float, 0x27800000u ^ split_flip(s ^ (int(threadIdx.x) & unpaired)));
+    const float odd =
+        __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, even) ^ split_flip(unpaired));
     constexpr int kPart[6][2] = {{1, 1}, {2, 0}, {0, 2}, {0, 1}, {1, 0}, {0, 0}};
     constexpr int SUMS = 2;
     bf16x8 fb[3][FN];
@@ -257,7 +260,7 @@ __device__ __forceinline__ void split_products(floatx4 (&acc)[FM][FN], const cha
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
                     acc[i][j0 + j][r] =
-                        __builtin_fmaf(t[j][r], r % 2 ? -unscale : unscale, acc[i][j0 + j][r]);
+                        __builtin_fmaf(t[j][r], r % 2 ? odd : even, acc[i][j0 + j][r]);
         }
     }
 }
@@ -417,10 +420,13 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
         if (k_begin < m0) k_begin = k_end < m0 ? k_end : m0;
     }
 
-    // The signs of the steps count from the chunk's first k, so that a product that skips k
-    // keeps those of the product that does not (BM and the chunks are multiples of a step).
-    const int step0 = __builtin_amdgcn_readfirstlane(
-        int((k_begin - int64_t(split) * g.k_chunk) / kSplitBK));
+    // The signs go by the chunk and count its steps from its first k, so that a product that
+    // skips k keeps those of the product that does not (BM and the chunks are multiples of a
+    // step). The chunk's pairs are even in number of steps, so this, the first step after them
+    // counted from k_begin, is odd where k_begin lies an odd number of steps into the chunk.
+    const int64_t chunk0 = int64_t(split) * g.k_chunk;
+    const int pairs = __builtin_amdgcn_readfirstlane(
+        split_pairs(min(g.k - chunk0, g.k_chunk)) - int((k_begin - chunk0) / kSplitBK));
 
     const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
     const int wm0 = (wave / (BN / WN)) * WM, wn0 = (wave % (BN / WN)) * WN;
@@ -468,10 +474,12 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
             tb.load_tail(pb + s * db, g.ldb, g.n - n0, left);
         }
     };
-    const auto convert = [&](int s) {
+    // `unpaired` masks the rows' and columns' signs: none in the steps that the unguarded loops
+    // below run, which leave the last two whole steps (a single stage: one) to those after them.
+    const auto convert = [&](int s, int unpaired) {
         char* st = lds + (STAGES == 2 ? (s & 1) * kStage : 0);
-        ta.store(st, split_scale(0));
-        tb.store(st + 3 * A::kPlane, split_scale(step0 + s));
+        ta.store(st, split_scale(A::row(0) & unpaired));
+        tb.store(st + 3 * A::kPlane, split_scale((s + pairs) ^ (B::row(0) & unpaired)));
         if constexpr (COLSUM) {
 #pragma unroll
             for (int u = 0; u < B::kUnits; ++u) {
@@ -480,12 +488,14 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
             }
         }
     };
-    const auto multiply = [&](int s) {
+    const auto multiply = [&](int s, int unpaired) {
         const char* st = lds + (STAGES == 2 ? (s & 1) * kStage : 0);
         split_products<FM, FN, A::kPlane, B::kPlane>(
             acc, st + (wm0 / 16) * 1024 + fbase,
-            st + 3 * A::kPlane + (wn0 / 16) * 1024 + fbase, step0 + s);
+            st + 3 * A::kPlane + (wn0 / 16) * 1024 + fbase, s + pairs, unpaired);
     };
+
+    const auto unpaired = [&](int s) { return s >= pairs ? -1 : 0; };
 
     // Two stages: while a step's products run, the next step is converted into the other stage
     // and the one after it loaded. One stage: the waves of the CU's other workgroups fill the
@@ -493,20 +503,20 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
     if constexpr (STAGES == 2) {
         if (steps > 0) {
             load_any(0);
-            convert(0);
+            convert(0, unpaired(0));
             if (steps > 1) load_any(1);
             __syncthreads();
         }
         int s = 0;
         for (; s + 2 < full; ++s) {
-            multiply(s);
-            convert(s + 1);
+            multiply(s, 0);
+            convert(s + 1, 0);
             load(s + 2);
             __syncthreads();
         }
         for (; s < steps; ++s) {
-            multiply(s);
-            if (s + 1 < steps) convert(s + 1);
+            multiply(s, unpaired(s));
+            if (s + 1 < steps) convert(s + 1, unpaired(s + 1));
             if (s + 2 < steps) load_any(s + 2);
             __syncthreads();
         }
@@ -514,17 +524,17 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
         if (steps > 0) load_any(0);
         int s = 0;
         for (; s + 1 < full; ++s) {
-            convert(s);
+            convert(s, 0);
             load(s + 1);
             __syncthreads();
-            multiply(s);
+            multiply(s, 0);
             __syncthreads();
         }
         for (; s < steps; ++s) {
-            convert(s);
+            convert(s, unpaired(s));
             if (s + 1 < steps) load_any(s + 1);
             __syncthreads();
-            multiply(s);
+            multiply(s, unpaired(s));
             __syncthreads();
         }
     }

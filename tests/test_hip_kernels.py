@@ -1291,10 +1291,10 @@ def test_staged_products_of_wide_ranges(hip, ta, tb, m, n, k):
 def test_staged_products_are_unbiased(hip, ta, tb, k, positive):
     """Rounding that takes neither side: over 2048 x 2048 results of independent errors the mean
     error is normal with the errors' rms over 2048, and over a column's 2048 with the rms over
-    sqrt(2048). Six times the first, and the columns' rms within a quarter of the second (2048
-    columns: its own standard deviation is 1.6 %, shared operands correlate it a little). Where
-    every product is positive, the losses of plain and negated sums differ a little: 2^-32 of
-    the results, a 256th of the last bit."""
+    sqrt(2048). Six times the first. Twice the second: of a pair of steps, a column's sums share
+    what the difference of its operands' sizes in the two leaves (1.5 measured at two pairs; with
+    one side taken throughout it is 15 and more). Where every product is positive, the losses of
+    plain and negated sums differ a little: 2^-32 of the results, a 256th of the last bit."""
     import torch
     print_case("staged bias", ta, tb, k, positive)
     g = torch.Generator(device="cuda").manual_seed(k)
@@ -1310,7 +1310,7 @@ def test_staged_products_are_unbiased(hip, ta, tb, k, positive):
     mean, column = abs(float(err.mean())), float((err.mean(0) ** 2).mean().sqrt())
     one_sign = 2.0 ** -32 * float((want * want).mean().sqrt()) if positive else 0.0
     assert mean <= 6 * rms / 2048 + one_sign, (mean * 2048 / rms)
-    assert column <= 1.25 * rms / 2048 ** 0.5, (column * 2048 ** 0.5 / rms)
+    assert column <= 2 * rms / 2048 ** 0.5, (column * 2048 ** 0.5 / rms)
 
 
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
