@@ -322,9 +322,9 @@ int launch_kslice(GemmArgs g, int64_t batch, hipStream_t s) {
 //      the larger tiles to fill the chip (512^3, the char-Transformer's layers)
 //   U  products of K's sizes that staged tiles do faster, K unsplit: like K's they
 //      use no workspace, which overlapping calls on several streams would share
-//   P   16 x 16 per workgroup of 16 waves, each wave a sixteenth of K: A^T B
-//       products of few tiles over a long K (weight gradients of narrow
-//       layers), one load round trip per 128 k of a wave, no workspace
+//   P  16 x 16 per workgroup of kPanelWaves waves, each a part of K: A^T B products of few
+//      tiles over a long K (weight gradients of narrow layers), one load round trip per 128 k
+//      of a wave, no workspace
 // A tile size is taken when its grid fills the 256 CUs (with split-K where K
 // is long) and the padding it adds to the output stays small.
 enum class Tile { L, M, S, K, T, U, P };

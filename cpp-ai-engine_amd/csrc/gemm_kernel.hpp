@@ -1,6 +1,7 @@
-// gemm_kernel.hpp -- the fp32 MFMA GEMM kernel templates (tile loaders, the
-// main kernel, the split-K reduction), shared by the dispatcher in gemm.hip.
-// See gemm.hip for the design.
+// gemm_kernel.hpp -- what the GEMM kernels share (arguments, epilogue) and the
+// fp32 MFMA ones: the K-sliced tiles, and the tile parts (Cfg, store_tile,
+// mfma_stage, store_acc) of the convolution gather kernels in conv_gemm.hip.
+// The staged products on bf16 parts are in gemm_split.hpp; gemm.hip chooses.
 #ifndef EHIP_GEMM_KERNEL_HPP
 #define EHIP_GEMM_KERNEL_HPP
 
@@ -128,8 +129,7 @@ __device__ __forceinline__ void store_tile(float* __restrict__ s, const float4* 
 // from LDS while the MFMAs of kk run (two register sets). Tiles of at most
 // 128 x 128 run four or more waves per SIMD: there the wave issuing its MFMAs
 // also takes priority over the others' loads and LDS traffic, which keeps the
-// matrix pipe fed (measured on MI355X: 5-9% on 8192 x 1024 x K; neither
-// change helps the 256 x 256 tile, nor priority alone).
+// matrix pipe fed.
 template <class C, int BK>
 __device__ __forceinline__ void mfma_stage(floatx16 (&acc)[C::kFM][C::kFN], const float* lds_a,
                                            const float* lds_b, int wm0, int wn0, int lane) {

@@ -1,6 +1,8 @@
 // gemm_split.hpp -- the staged-tile GEMM: fp32 products on the bf16 matrix instructions. Each
 // fp32 operand is the exact sum of three bf16 values, and the product is formed from six of the
-// nine products of the parts, accumulated in fp32.
+// nine products of the parts, accumulated in fp32: the three-way split of Henry, Tang and Heinecke
+// ("Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations",
+// ARITH 2019).
 //
 // 2^24 x = h + m + l, each the round-to-nearest bf16 of what is left: 24 significand bits in
 // 3 x 8. The last bit of an fp32 value is 2^-149 or more, so every part that is not zero is at
@@ -14,14 +16,14 @@
 // Error, against 64-bit products (2-norms; normal operands): K = 64 4.6e-8, K = 1024 1.13e-7,
 // K = 4096 2.1e-7, where the chain of v_mfma_f32_32x32x2f32 that it replaces has 1.4e-7, 5.7e-7
 // and 1.15e-6 (half-normal operands, half of them zero: 4.4e-8, 1.12e-7, 2.1e-7 against 1.0e-7,
-// 4.0e-7 and 8.1e-7); the mean over a column of 2048 is off by 1.0e-9 of the results' rms at K = 64
-// and 2.0e-9 at K = 1024, against 3.3e-9 and 9.2e-9. A step's 32 k are summed apart from the
+// 4.0e-7 and 8.1e-7); the mean over a column of 2048 is off by 1.8e-9 of the results' rms at K = 64
+// and 2.4e-9 at K = 1024, against 3.3e-9 and 9.2e-9. A step's 32 k are summed apart from the
 // accumulator (split_products) and their losses made to cancel (split_flip); all nine part products
 // would give the same figures.
 //
 // What bounds it: the matrix pipe at the clock the chip sustains. The bare instruction reaches
 // 1,950 TFLOP/s of its 2,500, i.e. 325 fp32 TFLOP/s with six products; 8192 x 1024 x 4096 runs
-// 217-221 (fp32 instructions: 127-131), the conversion and the sums taking about half of the
+// 192-219 by box (fp32 instructions: 127-131), the conversion and the sums taking about half of the
 // issue slots beside it. Measured and left out: the 32 x 32 x 16 instruction (212-227 where this
 // one, without the sums apart, has 222-236), the conversion before or after the products by
 // halves of the waves (200-207), raised priority around the products (216-232), loads two steps
@@ -608,7 +610,8 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
 
 // The staged tiles' shapes (gemm_kernel). per_cu: how many of a shape's workgroups a CU holds
 // (LDS and registers); rate: the throughput of a full CU relative to the first shape's,
-// measured on MI355X at 8192 x 1024 x 4096 (217-221, 197, 171 and 152 TFLOP/s).
+// measured on MI355X at 8192 x 1024 x 4096 (217-221, 197, 171 and 152 TFLOP/s on one box, before
+// the operands were scaled).
 struct TileShape {
     int bm, bn, per_cu;
     double rate;

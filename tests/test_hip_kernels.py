@@ -1127,39 +1127,43 @@ def test_gemm_probe(hip):
         hip.gemm_probe_read()
 
 
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("m,n,k,epi", [(8192, 1024, 1024, "plain"), (4096, 1024, 384, "beta"),
-                                       (4096, 2048, 256, "residual")])
-def test_nt_pipeline_matches_staged_tiles(hip, m, n, k, epi):
-    """A B^T of batch 1 in whole 128 x 128 tiles runs gemm_nt_pipe; the same product as
-    both entries of a batch of two (operand strides 0) runs the staged tiles, which the
-    pipeline's MFMA chain repeats: the outputs agree bit for bit, plain, with beta = 1 and
-    with a residual in the epilogue (shapes that neither batch splits along K)."""
+                                       (4096, 2048, 256, "residual"), (2560, 1024, 1024, "plain"),
+                                       (2560, 1024, 96, "beta")])
+def test_staged_tile_shapes_agree(hip, ta, tb, m, n, k, epi):
+    """A product alone and as each entry of a batch of two and of three (operand strides 0), none
+    of which splits K, agrees bit for bit, plain, with beta = 1 and with a residual in the
+    epilogue: the tile's shape does not change a bit. The last two sizes take 64 x 64, 128 x 64
+    and then 256 x 128 (K = 1024) or 128 x 128 (K = 96) tiles in batches of one, two and three."""
     import torch
     from ehip import GemmEx
-    print_case("nt pipeline vs staged", m, n, k, epi)
+    print_case("staged shapes", ta, tb, m, n, k, epi)
     g = torch.Generator(device="cuda").manual_seed(m + n + k)
-    a = torch.randn(m, k, device="cuda", generator=g)
-    b = torch.randn(n, k, device="cuda", generator=g)
+    a = torch.randn((k, m) if ta else (m, k), device="cuda", generator=g)
+    b = torch.randn((n, k) if tb else (k, n), device="cuda", generator=g)
     c0 = torch.randn(m, n, device="cuda", generator=g)
     res = torch.randn(m, n, device="cuda", generator=g)
     outs = []
-    for batch in (1, 2):
+    for batch in (1, 2, 3):
         c = c0.repeat(batch, 1).contiguous()
         d = GemmEx()
-        d.trans_a, d.trans_b, d.batch, d.inner = 0, 1, batch, 1
+        d.trans_a, d.trans_b, d.batch, d.inner = int(ta), int(tb), batch, 1
         d.m, d.n, d.k = m, n, k
-        d.a, d.lda, d.stride_a = hip.p(a), k, 0
-        d.b, d.ldb, d.stride_b = hip.p(b), k, 0
+        d.a, d.lda, d.stride_a = hip.p(a), a.shape[1], 0
+        d.b, d.ldb, d.stride_b = hip.p(b), b.shape[1], 0
         d.c, d.ldc, d.stride_c = hip.p(c), n, m * n
         d.alpha, d.addend_period = 1.0, 1
         d.beta = 1.0 if epi == "beta" else 0.0
         if epi == "residual" and batch == 1:
             d.residual, d.ld_residual = hip.p(res), n
         hip.gemm_ex(d)
-        if epi == "residual" and batch == 2:
-            c[:m] += res  # the separate add the epilogue replaces
-        outs.append(host(c[:m]))
-    exact(outs[0], outs[1], f"pipeline vs staged ({epi})")
+        for z in range(batch):
+            if epi == "residual" and batch > 1:
+                c[z * m:(z + 1) * m] += res  # the separate add the epilogue replaces
+            outs.append(host(c[z * m:(z + 1) * m]))
+    for z, out in enumerate(outs[1:]):
+        exact(out, outs[0], f"entry {z} ({epi})")
 
 
 # Staged products at the edges of their tiles: sizes one off the 64-, 128- and 256-element tiles,
