@@ -597,10 +597,10 @@ int ehip_conv2d_backward_weight_f32(const float* x, const float* grad_out, float
  *     cols; dbias = sum of grad_out per channel. Each output may be NULL to
  *     skip it; the ones given are overwritten.
  * Fixed-order sums (K split into fixed chunks on small grids): deterministic,
- * within the K-term tolerance of the reference's serial loops. Forward and
- * stride-1 dx of 24 or more gathered channels repack the weights into a block
- * of the arena when `stream` is NULL (calls on other streams gather without
- * one; both are within the same tolerance, not the same bits). Layers with
+ * within the K-term tolerance of the reference's serial loops. Large layers'
+ * forward and stride-1 dx repack the weights into a block of the arena when
+ * `stream` is NULL; calls on other streams, and those that find no block, read
+ * them as they are, for the same bits. Layers with
  * more than 2^31 - 1 elements in one image's input, output or weight rows, or
  * more than 65535 images, are refused with EHIP_EINVAL;
  * ehip_conv2d_igemm_supported() says 1 for a layer inside those limits (a
