@@ -628,8 +628,9 @@ __global__ __launch_bounds__(C::kThreads) void conv_dx_phase_kernel(GemmArgs g, 
 //   forward, dx  The reduction runs tap by tap, 32 channels of one tap per K step, so a thread's
 //     eight elements are eight channels of one input pixel: one bounds test and one offset per
 //     pixel and tap, the channels at a scalar stride. dx is the same product over dOut with
-//     the taps reversed and the padding kH - 1 - pad. The weights are repacked to match,
-//     (row, tap, channel) with the channels contiguous (one launch over a few hundred KB).
+//     the taps reversed and the padding kH - 1 - pad. The weights are read as they are
+//     (WeightTaps) or, where that pays and a block is to be had, repacked to match: (row, tap,
+//     channel) with the channels contiguous (PackedRows, one launch over a few hundred KB).
 //   dW  The reduction runs over the batch's output pixels; a thread's eight elements are eight
 //     consecutive pixels, decomposed once per step for all its rows (taps).
 //
