@@ -157,15 +157,17 @@ struct SplitTile {
     }
     // The same for a tile of which only the first `left` k are in the matrix (zeros after
     // them), with 64-bit offsets: the last step of a K that is no multiple of 32, and every
-    // step where a leading dimension is too large for offsets(). Units wholly inside load as
-    // above (KC): a K of 16 or 24 is one such step (18 x 242 x 242 x 16, A B^T: 9.0 -> 6.9 us).
+    // step where a leading dimension is too large for offsets(). KC: units wholly inside load as
+    // above (a K of 16 or 24 is one such step: 18 x 242 x 242 x 16, A B^T, 9.0 -> 6.9 us), those
+    // wholly outside not at all. Otherwise k past the last read the first again, for mask_tail to
+    // zero once the loads have been waited for.
     __device__ __forceinline__ void load_tail(global_bytes base, int64_t ld, int64_t rows_left,
                                               int left) {
 #pragma unroll
         for (int u = 0; u < kUnits; ++u) {
             const int64_t r = row(u) < rows_left ? row(u) : rows_left - 1;
-            const int in = left - 8 * group(u);
             if constexpr (KC) {
+                const int in = left - 8 * group(u);
                 const global_bytes p = base + 4 * (r * ld + 8 * group(u));
 #pragma unroll
                 for (int j = 0; j < 8; ++j) v[u][j] = 0.0f;
@@ -187,11 +189,19 @@ struct SplitTile {
             } else {
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    const int64_t k = j < in ? 8 * group(u) + j : 0;
-                    const float x = global_load<float>(base + 4 * (k * ld + r));
-                    v[u][j] = j < in ? x : 0.0f;
+                    const int k = 8 * group(u) + j;
+                    v[u][j] = global_load<float>(base + 4 * ((k < left ? k : 0) * ld + r));
                 }
             }
+        }
+    }
+    __device__ __forceinline__ void mask_tail(int left) {
+        if constexpr (!KC) {
+#pragma unroll
+            for (int u = 0; u < kUnits; ++u)
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    v[u][j] = 8 * group(u) + j < left ? v[u][j] : 0.0f;
         }
     }
     // Splits the registers, times `scale` (split_scale), into the three planes. A thread's units
@@ -467,13 +477,21 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
         ta.load(TA ? scalar(pa + s * da) : pa + s * da, oa, g.lda);
         tb.load(TB ? pb + s * db : scalar(pb + s * db), ob, g.ldb);
     };
+    const auto left = [&](int s) {
+        return int(min(k_end - k_begin - int64_t(s) * kSplitBK, int64_t(kSplitBK)));
+    };
     const auto load_any = [&](int s) {
         if (s < full) {
             load(s);
         } else {
-            const int left = int(min(k_end - k_begin - int64_t(s) * kSplitBK, int64_t(kSplitBK)));
-            ta.load_tail(pa + s * da, g.lda, g.m - m0, left);
-            tb.load_tail(pb + s * db, g.ldb, g.n - n0, left);
+            ta.load_tail(pa + s * da, g.lda, g.m - m0, left(s));
+            tb.load_tail(pb + s * db, g.ldb, g.n - n0, left(s));
+        }
+    };
+    const auto mask = [&](int s) {
+        if (s >= full) {
+            ta.mask_tail(left(s));
+            tb.mask_tail(left(s));
         }
     };
     // `unpaired` masks the rows' and columns' signs: none in the steps that the unguarded loops
@@ -505,6 +523,7 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
     if constexpr (STAGES == 2) {
         if (steps > 0) {
             load_any(0);
+            mask(0);
             convert(0, unpaired(0));
             if (steps > 1) load_any(1);
             __syncthreads();
@@ -518,7 +537,10 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
         }
         for (; s < steps; ++s) {
             multiply(s, unpaired(s));
-            if (s + 1 < steps) convert(s + 1, unpaired(s + 1));
+            if (s + 1 < steps) {
+                mask(s + 1);
+                convert(s + 1, unpaired(s + 1));
+            }
             if (s + 2 < steps) load_any(s + 2);
             __syncthreads();
         }
@@ -533,6 +555,7 @@ __global__ __launch_bounds__((TileThreads<BM, BN, WM, WN>::value), MINW) void ge
             __syncthreads();
         }
         for (; s < steps; ++s) {
+            mask(s);
             convert(s, unpaired(s));
             if (s + 1 < steps) load_any(s + 1);
             __syncthreads();
